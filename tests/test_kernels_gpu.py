@@ -176,6 +176,42 @@ def test_prompt_gemm_real_shapes(gpu, type_, rows, cols, batch):
         gpu.destroy(buf)
 
 
+# every token-block count of the GEMM (16, 32, 64, two of 64) and its edges, widths whose last
+# 128-column unit is half full, and rows that end inside a row tile
+@pytest.mark.parametrize("type_,rows,cols", [(Q4_K, 130, 768), (Q5_K, 17, 256), (Q6_K, 144, 1280), (Q8_0, 129, 320),
+                                             (Q4_0, 31, 64), (Q8_0, 16, 1152)])
+def test_prompt_gemm_batch_edges(gpu, type_, rows, cols):
+    rng = np.random.default_rng(rows + cols)
+    w = GEN[type_](rng, rows * cols // QUANTS[type_]["block"])
+    wb = gpu.upload_weights(type_, cols, rows, w)
+    for batch in (2, 15, 16, 17, 32, 33, 64, 65, 128, 129):
+        # magnitudes far apart between tokens and between columns: the split is scaled per token and 128 columns
+        x = rng.standard_normal((batch, cols)) * 10.0 ** rng.uniform(-6, 4, (batch, 1)) * 10.0 ** rng.uniform(-3, 3, cols)
+        x[batch // 2] = 0
+        x = x.astype(np.float32)
+        want = orc.matmul(type_, w, x.ravel(), cols, rows, rows, 0, 0, batch).reshape(batch, rows)
+        xb, yb = gpu.upload(x, "x"), gpu.buffer(batch * rows * 4, "y")
+        gpu.matmul(type_, wb, xb, yb, cols, rows, rows, 0, 0, batch)
+        got = gpu.read_f32(yb, batch * rows).reshape(batch, rows)
+        # a sum of cols f32 products in any order: cols * 2^-24 of the sum of magnitudes, which
+        # |w| <= 0.5 of these generators bounds by |x| / 2; 22-bit operands add 2^-21 of it
+        bound = (cols * 2.0 ** -24 + 2.0 ** -21) * 0.5 * np.abs(x.astype(np.float64)).sum(1, keepdims=True)
+        assert np.all(np.abs(got - want) <= bound), f"{type_} batch {batch}: {np.max(np.abs(got - want) / np.maximum(bound, 1e-30))}"
+        for buf in (xb, yb):
+            gpu.destroy(buf)
+    # an infinity stays in its token
+    x = rng.standard_normal((20, cols)).astype(np.float32)
+    x[7, 3] = np.inf
+    want = orc.matmul(type_, w, x.ravel(), cols, rows, rows, 0, 0, 20).reshape(20, rows)
+    xb, yb = gpu.upload(x, "x"), gpu.buffer(20 * rows * 4, "y")
+    gpu.matmul(type_, wb, xb, yb, cols, rows, rows, 0, 0, 20)
+    got = gpu.read_f32(yb, 20 * rows).reshape(20, rows)
+    assert not np.any(np.isfinite(got[7]))
+    near(np.delete(got, 7, 0), np.delete(want, 7, 0), 1e-4, "tokens beside an infinity")
+    for buf in (wb, xb, yb):
+        gpu.destroy(buf)
+
+
 # ---------------------------------------------------------------- verify.ts:39-54
 @pytest.mark.parametrize("window", [2, 16])
 def test_attention_small(gpu, window):

@@ -148,7 +148,7 @@ __global__ __launch_bounds__(256) void k_attention(AttnK a) {
 // With xs set (hd % 8 == 0, heads * hd % 64 == 0), the output row is also written in the
 // prompt GEMM's split form for the O projection (row = token * heads + head).
 __global__ __launch_bounds__(128) void k_attention_combine(const float *part, float *y, uint32_t rows,
-                                                           uint32_t hd, uint32_t nsplit, uint16_t *xs, uint32_t heads) {
+                                                           uint32_t hd, uint32_t nsplit, uint8_t *xs, uint32_t heads) {
   __shared__ float out[512];
   const uint64_t row = blockIdx.x;
   const uint64_t stride = (uint64_t)rows * (hd + 2);
@@ -182,7 +182,7 @@ __global__ __launch_bounds__(128) void k_attention_combine(const float *part, fl
 // past the last split, which selects leave out).
 template <uint32_t S>
 __global__ __launch_bounds__(128) void k_attention_combine_s(const float *part, float *y, uint32_t rows, uint32_t hd,
-                                                             uint32_t nsplit, uint16_t *xs, uint32_t heads) {
+                                                             uint32_t nsplit, uint8_t *xs, uint32_t heads) {
   __shared__ float out[512];
   const uint64_t row = blockIdx.x;
   const uint64_t stride = (uint64_t)rows * (hd + 2);
@@ -229,7 +229,7 @@ __global__ __launch_bounds__(128) void k_attention_combine_s(const float *part, 
 // The merge of nsplit key splits: the load-batched kernel when the splits fit it, else the
 // general one.
 static void launch_attention_combine(hipStream_t s, const float *part, float *y, uint32_t rows, uint32_t hd,
-                                     uint32_t nsplit, uint16_t *xs, uint32_t heads) {
+                                     uint32_t nsplit, uint8_t *xs, uint32_t heads) {
   const bool fits = (uint64_t)nsplit * rows * (hd + 2) * 4 < (1ull << 31);
   if (fits && nsplit <= 4)
     hipLaunchKernelGGL(k_attention_combine_s<4>, dim3(rows), dim3(128), 0, s, part, y, rows, hd, nsplit, xs, heads);
@@ -397,7 +397,7 @@ static hipError_t launch_attn_prompt(hipStream_t s, AttnK a, const AttnArgs &in,
   hipLaunchKernelGGL((k_attn_prompt<HD, E>), dim3(in.kv_heads, (nqt * a.group + 3) / 4, nsplit), dim3(256), lds, s, a);
   WGD_HIP(hipGetLastError());
   if (nsplit > 1) {
-    uint16_t *xs = in.xs && in.hd % 8 == 0 && in.heads * in.hd % 64 == 0 ? in.xs : nullptr;
+    uint8_t *xs = in.xs && in.hd % SPLIT_K == 0 ? in.xs : nullptr;
     launch_attention_combine(s, (const float *)in.partial, in.y, in.batch * in.heads, in.hd, nsplit, xs, in.heads);
     WGD_HIP(hipGetLastError());
     if (in.xs_written) *in.xs_written = xs != nullptr;

@@ -1,17 +1,15 @@
-// gemm.hip — prompt-batch dequant-GEMM on bf16 MFMA (gfx950).
+// gemm.hip — prompt-batch dequant-GEMM on the matrix cores (gfx950).
 //
 // The batched form of matmulShader (src/core/shaders.ts:39-54, dispatched with
 // batch = prompt chunk by engine.ts:130): y[b*stride + rowBase + r] = sum_c W[r][c] x[b+off][c].
-// It is a real dense contraction, so it runs on v_mfma_f32_16x16x32_bf16. bf16 keeps 8
-// significant bits, which alone would cost ~2^-9 relative error per output and break the
-// 1e-3 logits bound, so both operands are split: v = hi + lo with hi = RN_bf16(v),
-// lo = RN_bf16(v - hi), and the product is accumulated as hi*hi + hi*lo + lo*hi in f32
-// (relative error ~2^-16). Weights are dequantized from their GGUF (or planar) blocks
-// straight into MFMA operand registers; the activation tile is split once into LDS.
+// It is a real dense contraction, so it runs on MFMA. 16-bit operands alone would break the
+// 1e-3 logits bound, so operands are split into (hi, lo) pairs.
 //
-// Tiling: a workgroup (4 wavefronts) owns 64 rows x 64 tokens; each wavefront owns
-// 16 rows x 64 tokens = four 16x16 accumulator tiles; K advances 32 per MFMA step and
-// 64 per LDS tile.
+// k_gemm (GGUF-layout weights, F16, F32) splits both sides into bf16 pairs, hi = RN_bf16(v),
+// lo = RN_bf16(v - hi), and sums hi*hi + hi*lo + lo*hi in f32 (relative error ~2^-16). A
+// workgroup (4 wavefronts) owns 64 rows x 64 tokens; each wavefront owns 16 rows x 64
+// tokens = four 16x16 accumulator tiles; K advances 32 per MFMA step and 64 per LDS tile.
+// k_gemm_q (planar weights) is described at its definition below.
 #include "internal.h"
 #include "decode.h"
 #include "split.h"
@@ -225,26 +223,37 @@ __global__ __launch_bounds__(256) void k_gemm(GemmArgs a) {
   }
 }
 
-// ------------------------------------------------------------------ planar K-quant GEMM
+// ------------------------------------------------------------------ planar quant GEMM
 //
-// The prompt GEMM of the planar layouts (Q4_K, Q5_K, Q6_K, Q8_0, Q4_0; the decode matvec's weights). A
-// workgroup owns QG_M = 128 weight rows x QG_N = 128 tokens and a K span (split-K when the
-// rows alone give too few workgroups; partial sums are added in split order by
-// k_gemm_reduce, so results do not depend on timing). The activations are split into bf16
-// (hi, lo) once per input by k_gemm_split, already in MFMA fragment order, so each
-// wavefront loads its activation fragments of a K tile straight from that buffer (L2
-// hits: every workgroup of the launch reads the same tiles) into registers, 1 KB per load
-// instruction, before the tile's dequantization. Per 64-column K tile every weight of the
-// workgroup's rows is dequantized once, from coalesced 16-byte planar loads (one 32-element
-// chunk of one row per thread), split the same way and stored in LDS in fragment order.
-// Four wavefronts each compute 64 rows x 64 tokens, sixteen 16 x 16 accumulators, three
-// MFMAs per product (hi*hi + hi*lo + lo*hi). The next K tile's weight loads are issued
-// before the MFMAs of the current one; two workgroups share a CU (the register budget of
-// the launch bounds), so one's dequantization can run beside the other's MFMAs.
+// The prompt GEMM of the planar layouts (Q4_K, Q5_K, Q6_K, Q8_0, Q4_0; the decode matvec's
+// weights). A workgroup owns QG_M = 128 weight rows x 16 TT tokens and a K span (split-K when
+// the rows alone give too few workgroups; partial sums are added in split order by the
+// finishes, so results do not depend on timing).
 //
-// The weight tile is kept in LDS in the activations' fragment order (split.h), as rows.
-constexpr uint32_t QG_M = 128, QG_N = SPLIT_N, QG_K = SPLIT_K, QG_TILE = SPLIT_TILE;
-constexpr uint32_t QG_LDS = QG_TILE * 2;  // bytes: weight tile
+// Every weight is unpacked once per workgroup, in registers, by the one wavefront that uses
+// it: lane 16 g + c loads the 32-element chunk g of row c of a 128-column unit (1 KB of
+// contiguous bytes a wavefront), and its four groups of eight are the B operands of four
+// v_mfma_f32_16x16x32_f16, each summing over one group of every chunk. The weights enter as exact
+// f16 integers: sc * q <= 63 * 31 for Q4_K and Q5_K, q for Q8_0 and Q4_0, and sc * (q - 32)
+// as an exact (hi, lo) pair for Q6_K. The activations are split.h's (hi, lo) pairs: two
+// MFMAs per product (three for Q6_K; its lo * lo part is below 2^-22 of the product). A unit's
+// sums are scaled by the row's d and the token's scale in f32, and the K-quants' min term,
+// -dmin * m times the sums of x, is one f32 MFMA (16x16x4: its four K entries are the unit's
+// four chunks). The worst errors against float64 are those of f32 sums (mlp of Q6_K 4096 x
+// 14336, 32 tokens: 2.8e-7 relative; bf16 pairs of both operands gave 6.9e-6).
+//
+// The activations go through two LDS buffers of S units: the next S units are loaded into
+// registers while the current ones are used, one barrier per S units. D units of weights are
+// in flight per row tile. Every load is issued without a branch around it (past the span it
+// reads through an empty resource), so each wait counts exactly the loads behind it.
+//
+// What it replaces: bf16 pairs of dequantized weights in LDS, always 128 tokens wide, three
+// MFMAs per product and about 210 VALU instructions per 32 weights against about 70. Kernel times
+// of the 8B shape, Q4_K: 16 tokens, gate + up (28672 x 4096) 86 -> 22 us, a prompt of 250
+// tokens in 16s over 4 layers 12.8 -> 6.2 ms; 128 tokens, gate + up 88 -> 83 us, down 47 ->
+// 41, Q/K/V 28.5 -> 27.
+constexpr uint32_t QG_M = 128, QG_K = 64;
+constexpr uint32_t QG_U = SPLIT_K;   // columns of a unit
 
 // One weight matrix of a grouped launch: its planar geometry, the row-tile count, and where
 // its rows go (y, or rows [row0, row0 + rows) of the group's split-K partial sums).
@@ -259,23 +268,17 @@ constexpr uint32_t QG_MAX_JOBS = 3;
 // over the concatenated row tiles; kind 0 / 1 selects the launch's first / second type.
 struct QGemm {
   QJob job[QG_MAX_JOBS]; uint32_t njobs;
-  const uint16_t *xs; float *part;
-  uint32_t cols, batch, kspan, rows_total, accumulate;
+  const uint8_t *xs; float *part;
+  uint32_t cols, batch, kspan, rows_total, accumulate;  // kspan: a multiple of QG_U
 };
 
-// Activations [batch][cols] f32 -> the split form (split.h); tokens past the batch up to the
-// tile are zero. One thread per eight consecutive columns of a token.
-__global__ __launch_bounds__(256) void k_gemm_split(const float *x, uint16_t *xs, uint32_t cols, uint32_t batch,
-                                                    uint32_t count) {
-  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= count) return;
-  const uint32_t c8 = cols / 8, tok = i / c8, k = (i % c8) * 8;
-  float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b = a;
-  if (tok < batch) {
-    a = *(const float4 *)(x + (uint64_t)tok * cols + k);
-    b = *(const float4 *)(x + (uint64_t)tok * cols + k + 4);
-  }
-  split_store8(xs, cols, tok, k, a, b);
+// Activations [batch][cols] f32 -> the split form (split.h): one thread per eight
+// consecutive columns of a token, 16 threads per 128 columns.
+__global__ __launch_bounds__(256) void k_gemm_split(const float *x, uint8_t *xs, uint32_t cols, uint32_t count) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x, c8 = split_kblocks(cols) * 16, tok = i / c8, k = (i % c8) * 8;
+  if (i >= count || k >= cols) return;
+  const float4 *p = (const float4 *)(x + (uint64_t)tok * cols + k);
+  split_store8(xs, cols, tok, k, p[0], p[1]);
 }
 
 typedef __amdgpu_buffer_rsrc_t QRsrc;
@@ -284,240 +287,350 @@ __device__ __forceinline__ uint4 qld16(QRsrc r, uint32_t off) {
   const u4 v = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
   return make_uint4(v.x, v.y, v.z, v.w);
 }
+__device__ __forceinline__ uint2 qld8(QRsrc r, uint32_t off) {
+  typedef unsigned int u2 __attribute__((ext_vector_type(2)));
+  const u2 v = __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0);
+  return make_uint2(v.x, v.y);
+}
+__device__ __forceinline__ uint32_t qld2(QRsrc r, uint32_t off) { return __builtin_amdgcn_raw_buffer_load_b16(r, off, 0, 0); }
 
-// One thread's weights of a K tile: Q4_K / Q6_K one 32-element chunk (row-tile rt, column
-// cc of the tile, row r), Q8_0 two 16-element chunks.
-template <int TYPE> struct QWeights;
-template <> struct QWeights<Q4_K> {
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+__device__ __forceinline__ f16x2 h2(uint32_t v) { return __builtin_bit_cast(f16x2, v); }
+__device__ __forceinline__ uint32_t u32(f16x2 v) { return __builtin_bit_cast(uint32_t, v); }
+__device__ __forceinline__ f16x2 both(_Float16 v) { return f16x2{v, v}; }
+__device__ __forceinline__ float f16_lo(uint32_t v) { return (float)__builtin_bit_cast(_Float16, (uint16_t)v); }
+// Bytes 0 and 2, and bytes 1 and 3, of a dword as 1024 + byte in f16 (the byte in the mantissa's
+// low bits): one byte permute each.
+__device__ __forceinline__ f16x2 bytes02(uint32_t v) { return h2(__builtin_amdgcn_perm(0x64646464u, v, 0x04020400u)); }
+__device__ __forceinline__ f16x2 bytes13(uint32_t v) { return h2(__builtin_amdgcn_perm(0x64646464u, v, 0x04030401u)); }
+// (v & mask) | bits as one instruction (the compiler keeps two where both are literals).
+__device__ __forceinline__ uint32_t and_or(uint32_t v, uint32_t mask, uint32_t bits) {
+  asm("" : "+s"(mask));
+  asm("" : "+v"(bits));
+  return (v & mask) | bits;
+}
+__device__ __forceinline__ f16x2 fma2(f16x2 a, f16x2 b, f16x2 c) { return __builtin_elementwise_fma(a, b, c); }
+__device__ __forceinline__ f16x8 oct(f16x2 a, f16x2 b, f16x2 c, f16x2 d) {
+  return __builtin_bit_cast(f16x8, make_uint4(u32(a), u32(b), u32(c), u32(d)));
+}
+// The 6-bit scale and min of the sub-block of chunk lane group g in unit parity odd (quant.ts:9-12).
+__device__ __forceinline__ void scale_min(const uint4 &h, uint32_t odd, uint32_t g, uint32_t &sc, uint32_t &m) {
+  const uint32_t sh = 8 * g, A = h.y >> sh, B = h.z >> sh, C = h.w >> sh;
+  const uint32_t o = 0u - odd;  // selects, not branches: odd is uniform and known only at run time
+  sc = (((C & 15u) | ((A >> 2) & 48u)) & o) | (A & 63u & ~o);
+  m = ((((C >> 4) & 15u) | ((B >> 2) & 48u)) & o) | (B & 63u & ~o);
+}
+
+// A lane's weights of 16 rows x one 128-column unit. fetch() loads them; unpack() leaves the MFMA
+// operands w[j] (wl[j]: their lo parts, LO types), for the types of whole 256-column blocks the row's d in d[0] and
+// the chunk's -dmin * m in mn (MIN types), for the 32-column block types block j's d in d[j].
+// CHUNK types: operand j holds elements 8 j .. + 8 of chunk g; else elements 8 g .. + 8 of block j.
+template <int TYPE> struct QUnit;
+template <> struct QUnit<Q4_K> {
+  static constexpr bool CHUNK = true, LO = false, MIN = true;
   uint4 q, h;
-  __device__ void fetch(const QJob &a, QRsrc rw, uint32_t T, uint32_t r, uint32_t c) {
-    q = qld16(rw, ((T * a.C + c) * 16 + r) * 16);
-    h = qld16(rw, a.nbp * 128 + ((T * a.bpr + c / 8) * 16 + r) * 16);
+  __device__ void fetch(const QJob &a, QRsrc rw, uint32_t T, uint32_t u, uint32_t g, uint32_t c) {
+    q = qld16(rw, ((T * a.C + 4 * u + g) * 16 + c) * 16);
+    h = qld16(rw, a.nbp * 128 + ((T * a.bpr + u / 2) * 16 + c) * 16);
   }
-  // element e < 32 of the chunk into f32 (quant.ts:13-19: d * sc * q - dmin * m)
-  __device__ void values(uint32_t c, float *v) const {
-    const uint32_t s = c & 7, sh = 8 * (s & 3);
+  __device__ void unpack(uint32_t u, uint32_t g, f16x8 *w, f16x8 *, float *d, float &mn) const {
     uint32_t sc, m;
-    if (s < 4) { sc = (h.y >> sh) & 63u; m = (h.z >> sh) & 63u; }
-    else { sc = ((h.w >> sh) & 15u) | (((h.y >> sh) >> 6 & 3u) << 4); m = ((h.w >> sh) >> 4 & 15u) | (((h.z >> sh) >> 6 & 3u) << 4); }
-    const float dsc = half_bits(h.x & 0xFFFFu) * (float)sc, dmm = half_bits(h.x >> 16) * (float)m;
-    const uint32_t qw[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-      const uint32_t lo = qw[k] & 0x0F0F0F0Fu, hi = (qw[k] >> 4) & 0x0F0F0F0Fu;
-#pragma unroll
-      for (int b = 0; b < 4; b++) {
-        v[4 * k + b] = fmaf(dsc, (float)((lo >> (8 * b)) & 0xFFu), -dmm);
-        v[16 + 4 * k + b] = fmaf(dsc, (float)((hi >> (8 * b)) & 0xFFu), -dmm);
-      }
-    }
+    scale_min(h, u & 1, g, sc, m);
+    d[0] = f16_lo(h.x);
+    mn = -f16_lo(h.x >> 16) * (float)m;
+    // low nibbles as 1024 + q, high nibbles (bits 4-7 of the mantissa, in units of 1/16 at 64) as 64 + q:
+    // sc * (1024 + q) - 1024 sc and sc * (64 + q) - 64 sc are exact, 1024 sc <= 64512
+    const f16x2 s = both((_Float16)(uint16_t)sc), bl = s * both((_Float16)-1024.f), bh = s * both((_Float16)-64.f);
+    auto lo = [&](uint32_t v) { return fma2(h2(and_or(v, 0x000F000Fu, 0x64006400u)), s, bl); };
+    auto hi = [&](uint32_t v) { return fma2(h2(and_or(v, 0x00F000F0u, 0x54005400u)), s, bh); };
+    const uint32_t x = q.x >> 8, y = q.y >> 8, z = q.z >> 8, t = q.w >> 8;
+    w[0] = oct(lo(q.x), lo(x), lo(q.y), lo(y));
+    w[1] = oct(lo(q.z), lo(z), lo(q.w), lo(t));
+    w[2] = oct(hi(q.x), hi(x), hi(q.y), hi(y));
+    w[3] = oct(hi(q.z), hi(z), hi(q.w), hi(t));
   }
 };
-template <> struct QWeights<Q6_K> {
-  uint4 q; uint2 qh; uint32_t sc, d;
-  __device__ void fetch(const QJob &a, QRsrc rw, uint32_t T, uint32_t r, uint32_t c) {
-    const uint32_t tc = (T * a.C + c) * 16 + r;
+// Q5_K: Q4_K's chunk and header planes (the header after the fifth-bit plane) and the
+// chunk's dword of fifth bits, moved to bit 4 of each quant byte.
+template <> struct QUnit<Q5_K> {
+  static constexpr bool CHUNK = true, LO = false, MIN = true;
+  uint4 q, h; uint32_t b;
+  __device__ void fetch(const QJob &a, QRsrc rw, uint32_t T, uint32_t u, uint32_t g, uint32_t c) {
+    const uint32_t tc = (T * a.C + 4 * u + g) * 16 + c;
     q = qld16(rw, tc * 16);
-    typedef unsigned int u2 __attribute__((ext_vector_type(2)));
-    const u2 hv = __builtin_amdgcn_raw_buffer_load_b64(rw, a.nbp * 128 + tc * 8, 0, 0);
-    qh = make_uint2(hv.x, hv.y);
-    sc = __builtin_amdgcn_raw_buffer_load_b16(rw, a.nbp * 192 + tc * 2, 0, 0);
-    d = __builtin_amdgcn_raw_buffer_load_b16(rw, a.nbp * 208 + ((T * a.bpr + c / 8) * 16 + r) * 2, 0, 0);
+    b = __builtin_amdgcn_raw_buffer_load_b32(rw, a.nbp * 128 + tc * 4, 0, 0);
+    h = qld16(rw, a.nbp * 160 + ((T * a.bpr + u / 2) * 16 + c) * 16);
   }
-  // quant.ts:21-27: d * scale16 * (q - 32); low nibbles with high bits at bits 4-5
-  __device__ void values(uint32_t, float *v) const {
-    const float d0 = half_bits(d & 0xFFFFu);
-    const float s0 = d0 * (float)(int8_t)(sc & 0xFFu), s1 = d0 * (float)(int8_t)((sc >> 8) & 0xFFu);
+  __device__ void unpack(uint32_t u, uint32_t g, f16x8 *w, f16x8 *, float *d, float &mn) const {
+    uint32_t sc, m;
+    scale_min(h, u & 1, g, sc, m);
+    d[0] = f16_lo(h.x);
+    mn = -f16_lo(h.x >> 16) * (float)m;
+    const f16x2 s = both((_Float16)(uint16_t)sc), bl = s * both((_Float16)-1024.f);
     const uint32_t qw[4] = {q.x, q.y, q.z, q.w};
+    f16x2 v[16];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const uint32_t lo = (qw[k] & 0x0F0F0F0Fu) | ((b << (4 - k)) & 0x10101010u);
+      const uint32_t hi = ((qw[k] >> 4) & 0x0F0F0F0Fu) | ((b >> k) & 0x10101010u);
+      v[2 * k] = fma2(bytes02(lo), s, bl);
+      v[2 * k + 1] = fma2(bytes13(lo), s, bl);
+      v[8 + 2 * k] = fma2(bytes02(hi), s, bl);
+      v[8 + 2 * k + 1] = fma2(bytes13(hi), s, bl);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) w[j] = oct(v[4 * j], v[4 * j + 1], v[4 * j + 2], v[4 * j + 3]);
+  }
+};
+// Q6_K: sc * (q - 32) has up to 12 bits; hi = RN_f16, lo = the exact rest.
+template <> struct QUnit<Q6_K> {
+  static constexpr bool CHUNK = true, LO = true, MIN = false;
+  uint4 q; uint2 qh; uint32_t sc, dd;
+  __device__ void fetch(const QJob &a, QRsrc rw, uint32_t T, uint32_t u, uint32_t g, uint32_t c) {
+    const uint32_t tc = (T * a.C + 4 * u + g) * 16 + c;
+    q = qld16(rw, tc * 16);
+    qh = qld8(rw, a.nbp * 128 + tc * 8);
+    sc = qld2(rw, a.nbp * 192 + tc * 2);
+    dd = qld2(rw, a.nbp * 208 + ((T * a.bpr + u / 2) * 16 + c) * 2);
+  }
+  __device__ void unpack(uint32_t, uint32_t, f16x8 *w, f16x8 *wl, float *d, float &) const {
+    d[0] = f16_lo(dd);
+    const f16x2 s0 = both((_Float16)(int16_t)(int8_t)sc), s1 = both((_Float16)(int16_t)(int8_t)(sc >> 8));
+    const f16x2 off = both((_Float16)-1056.f);
+    const uint32_t qw[4] = {q.x, q.y, q.z, q.w};
+    f16x2 v[16], r[16];
+    auto put = [&](int i, f16x2 n, f16x2 s) {
+      n += off;
+      v[i] = n * s;
+      r[i] = fma2(n, s, -v[i]);
+    };
 #pragma unroll
     for (int k = 0; k < 4; k++) {
       const uint32_t Q = (k < 2 ? qh.x : qh.y) >> (4 * (k & 1));
       const uint32_t lo = (qw[k] & 0x0F0F0F0Fu) | ((Q << 4) & 0x30303030u);
       const uint32_t hi = ((qw[k] >> 4) & 0x0F0F0F0Fu) | ((Q << 2) & 0x30303030u);
+      put(2 * k, bytes02(lo), s0);
+      put(2 * k + 1, bytes13(lo), s0);
+      put(8 + 2 * k, bytes02(hi), s1);
+      put(8 + 2 * k + 1, bytes13(hi), s1);
+    }
 #pragma unroll
-      for (int b = 0; b < 4; b++) {
-        v[4 * k + b] = s0 * (float)((int)((lo >> (8 * b)) & 0xFFu) - 32);
-        v[16 + 4 * k + b] = s1 * (float)((int)((hi >> (8 * b)) & 0xFFu) - 32);
-      }
+    for (int j = 0; j < 4; j++) {
+      w[j] = oct(v[4 * j], v[4 * j + 1], v[4 * j + 2], v[4 * j + 3]);
+      wl[j] = oct(r[4 * j], r[4 * j + 1], r[4 * j + 2], r[4 * j + 3]);
     }
   }
 };
-template <> struct QWeights<Q8_0> {
-  uint4 q[2]; uint32_t d[2];
-  // chunks 2c and 2c + 1 (16 elements each, one Q8_0 block): c counts 32-element columns
-  __device__ void fetch(const QJob &a, QRsrc rw, uint32_t T, uint32_t r, uint32_t c) {
+// Q8_0: block j of the unit is chunks 2 j, 2 j + 1 of 16 bytes; a lane takes eight of its bytes.
+template <> struct QUnit<Q8_0> {
+  static constexpr bool CHUNK = false, LO = false, MIN = false;
+  uint2 q[4]; uint32_t dd[4];
+  __device__ void fetch(const QJob &a, QRsrc rw, uint32_t T, uint32_t u, uint32_t g, uint32_t c) {
 #pragma unroll
-    for (int u = 0; u < 2; u++) q[u] = qld16(rw, ((T * a.C + 2 * c + u) * 16 + r) * 16);
-    d[0] = d[1] = __builtin_amdgcn_raw_buffer_load_b16(rw, a.nbp * 32 + ((T * a.bpr + c) * 16 + r) * 2, 0, 0);
+    for (uint32_t j = 0; j < 4; j++) {
+      q[j] = qld8(rw, ((T * a.C + 8 * u + 2 * j + (g >> 1)) * 16 + c) * 16 + 8 * (g & 1));
+      dd[j] = qld2(rw, a.nbp * 32 + ((T * a.bpr + 4 * u + j) * 16 + c) * 2);
+    }
   }
-  __device__ void values(uint32_t, float *v) const {
-    const float dd = half_bits(d[0] & 0xFFFFu);
+  __device__ void unpack(uint32_t, uint32_t, f16x8 *w, f16x8 *, float *d, float &) const {
+    const f16x2 off = both((_Float16)-1152.f);  // the sign bit flipped: byte + 128
 #pragma unroll
-    for (int u = 0; u < 2; u++) {
-      const uint32_t qw[4] = {q[u].x, q[u].y, q[u].z, q[u].w};
-#pragma unroll
-      for (int k = 0; k < 4; k++)
-#pragma unroll
-        for (int b = 0; b < 4; b++) v[16 * u + 4 * k + b] = dd * (float)(int8_t)((qw[k] >> (8 * b)) & 0xFFu);
+    for (int j = 0; j < 4; j++) {
+      const uint32_t x = q[j].x ^ 0x80808080u, y = q[j].y ^ 0x80808080u;
+      w[j] = oct(bytes02(x) + off, bytes13(x) + off, bytes02(y) + off, bytes13(y) + off);
+      d[j] = f16_lo(dd[j]);
     }
   }
 };
-
-// Q5_K: Q4_K's chunk and header planes (the header after the fifth-bit plane) and the
-// chunk's dword of fifth bits, moved to bit 4 of each quant byte (quant.ts:13-19).
-template <> struct QWeights<Q5_K> {
-  uint4 q, h; uint32_t b;
-  __device__ void fetch(const QJob &a, QRsrc rw, uint32_t T, uint32_t r, uint32_t c) {
-    const uint32_t tc = (T * a.C + c) * 16 + r;
-    q = qld16(rw, tc * 16);
-    b = __builtin_amdgcn_raw_buffer_load_b32(rw, a.nbp * 128 + tc * 4, 0, 0);
-    h = qld16(rw, a.nbp * 160 + ((T * a.bpr + c / 8) * 16 + r) * 16);
-  }
-  __device__ void values(uint32_t c, float *v) const {
-    const uint32_t s = c & 7, sh = 8 * (s & 3);
-    uint32_t sc, m;
-    if (s < 4) { sc = (h.y >> sh) & 63u; m = (h.z >> sh) & 63u; }
-    else { sc = ((h.w >> sh) & 15u) | (((h.y >> sh) >> 6 & 3u) << 4); m = ((h.w >> sh) >> 4 & 15u) | (((h.z >> sh) >> 6 & 3u) << 4); }
-    const float dsc = half_bits(h.x & 0xFFFFu) * (float)sc, dmm = half_bits(h.x >> 16) * (float)m;
-    const uint32_t qw[4] = {q.x, q.y, q.z, q.w};
+// Q4_0: block j is one chunk; lane group g takes bytes 8 (g % 2) .. + 8, nibble g / 2.
+template <> struct QUnit<Q4_0> {
+  static constexpr bool CHUNK = false, LO = false, MIN = false;
+  uint2 q[4]; uint32_t dd[4];
+  __device__ void fetch(const QJob &a, QRsrc rw, uint32_t T, uint32_t u, uint32_t g, uint32_t c) {
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-      const uint32_t lo = (qw[k] & 0x0F0F0F0Fu) | ((b << (4 - k)) & 0x10101010u);
-      const uint32_t hi = ((qw[k] >> 4) & 0x0F0F0F0Fu) | ((b >> k) & 0x10101010u);
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        v[4 * k + e] = fmaf(dsc, (float)((lo >> (8 * e)) & 0xFFu), -dmm);
-        v[16 + 4 * k + e] = fmaf(dsc, (float)((hi >> (8 * e)) & 0xFFu), -dmm);
-      }
+    for (uint32_t j = 0; j < 4; j++) {
+      const uint32_t tc = (T * a.C + 4 * u + j) * 16 + c;
+      q[j] = qld8(rw, tc * 16 + 8 * (g & 1));
+      dd[j] = qld2(rw, a.nbp * 16 + tc * 2);
     }
   }
-};
-// Q4_0: one block per chunk, d * (q - 8) (quant.ts:7).
-template <> struct QWeights<Q4_0> {
-  uint4 q; uint32_t d;
-  __device__ void fetch(const QJob &a, QRsrc rw, uint32_t T, uint32_t r, uint32_t c) {
-    const uint32_t tc = (T * a.C + c) * 16 + r;
-    q = qld16(rw, tc * 16);
-    d = __builtin_amdgcn_raw_buffer_load_b16(rw, a.nbp * 16 + tc * 2, 0, 0);
-  }
-  __device__ void values(uint32_t, float *v) const {
-    const float dd = half_bits(d & 0xFFFFu);
-    const uint32_t qw[4] = {q.x, q.y, q.z, q.w};
+  __device__ void unpack(uint32_t, uint32_t g, f16x8 *w, f16x8 *, float *d, float &) const {
+    const f16x2 off = both((_Float16)-1032.f);
+    const uint32_t sh = 4 * (g >> 1);
 #pragma unroll
-    for (int k = 0; k < 4; k++)
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        v[4 * k + e] = dd * (float)((int)((qw[k] >> (8 * e)) & 15u) - 8);
-        v[16 + 4 * k + e] = dd * (float)((int)((qw[k] >> (8 * e + 4)) & 15u) - 8);
-      }
+    for (int j = 0; j < 4; j++) {
+      const uint32_t x = (q[j].x >> sh) & 0x0F0F0F0Fu, y = (q[j].y >> sh) & 0x0F0F0F0Fu;
+      w[j] = oct(bytes02(x) + off, bytes13(x) + off, bytes02(y) + off, bytes13(y) + off);
+      d[j] = f16_lo(dd[j]);
+    }
   }
 };
 
-template <int TYPE>
-__device__ __forceinline__ void gemm_tile(const QGemm &a, const QJob &jb, uint32_t mt, uint16_t *qlds) {
-  uint16_t *wt = qlds;
-  const uint32_t tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, wm = wv & 1, wn = wv >> 1;
-  const uint32_t m0 = mt * QG_M, n0 = blockIdx.y * QG_N, z = blockIdx.z;
-  const uint32_t kb = z * a.kspan, ke = kb + a.kspan < a.cols ? kb + a.kspan : a.cols;
-  const QRsrc rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(jb.w), 0, (int)jb.wbytes, 0x00020000);
-  // this thread's weights: row tile wrt, 32-column half wcc of the K tile, row wr
-  const uint32_t wrt = tid >> 5, wcc = (tid >> 4) & 1, wr = tid & 15;
-  const uint32_t ktiles = a.cols / QG_K;
-  const QRsrc rx = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint16_t *>(a.xs + (uint64_t)blockIdx.y * ktiles * QG_TILE), 0, (int)(ktiles * QG_TILE * 2), 0x00020000);
-  QWeights<TYPE> wreg;
-  auto fetch = [&](uint32_t k0) { wreg.fetch(jb, rw, m0 / 16 + wrt, wr, k0 / 32 + wcc); };
-  // this wavefront's activation fragments of a K tile, from the split buffer
-  auto xfrag = [&](uint32_t k0, uint32_t hl, uint32_t b, uint32_t ks) {
-    return __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(
-        rx, 2 * ((k0 / QG_K) * QG_TILE + frag_at(hl, b, ks, 0, 0) + 8 * lane), 0, 0));
+// Row tiles per wavefront. Up to 32 tokens the weight stream is the bound, and eight
+// wavefronts of one row tile (128 registers or less, so four per SIMD) hide its latency better
+// than four of two (8B prompt in 16s 6.22 against 6.34 ms); for 64 tokens two row tiles halve
+// the LDS reads of the activations per MFMA.
+constexpr uint32_t qg_rt(uint32_t tt) { return tt <= 2 ? 1 : 2; }
+constexpr uint32_t qg_threads(uint32_t tt) { return QG_M / 16 / qg_rt(tt) * 64; }
+// Units of weights in flight per row tile (registers), and units of activations per LDS buffer (17 to 34 KB).
+constexpr uint32_t qg_depth(int type, uint32_t tt) { return type == Q8_0 || type == Q4_0 ? (tt <= 2 ? 2 : 1) : tt <= 2 ? 4 : 2; }
+constexpr uint32_t qg_stage(int type, uint32_t tt) { return 4 / tt < qg_depth(type, tt) ? 4 / tt : qg_depth(type, tt); }
+
+template <int TYPE, uint32_t TT>
+__device__ __forceinline__ void gemm_tile(const QGemm &a, const QJob &jb, uint32_t mt, uint8_t *lds) {
+  constexpr uint32_t RT = qg_rt(TT), D = qg_depth(TYPE, TT), S = qg_stage(TYPE, TT), UB = TT * SPLIT_BLOCK, NT = qg_threads(TT);
+  typedef QUnit<TYPE> W;
+  const uint32_t tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, g = lane >> 4, c = lane & 15;
+  const uint32_t m0 = mt * QG_M + wv * 16 * RT, b0 = blockIdx.y * TT, z = blockIdx.z;
+  const uint32_t kbs = split_kblocks(a.cols);
+  const uint32_t u0 = z * (a.kspan / QG_U), ue = u0 + a.kspan / QG_U, u1 = ue < kbs ? ue : kbs;
+  const uint32_t T0 = m0 / 16;
+  f32x4 acc[RT][TT];
+#pragma unroll
+  for (uint32_t r = 0; r < RT; r++)
+#pragma unroll
+    for (uint32_t t = 0; t < TT; t++) acc[r][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  W buf[D][RT];
+  // Units past the span read zeros (a resource of no bytes) and no memory: the loop below has
+  // no branch around a load or its use, so the waits count exactly the loads behind them.
+  auto fetch = [&](uint32_t d, uint32_t u) {
+    const QRsrc rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(jb.w), 0, u < u1 ? (int)jb.wbytes : 0, 0x00020000);
+#pragma unroll
+    for (uint32_t r = 0; r < RT; r++) buf[d][r].fetch(jb, rw, T0 + r, u, g, c);
   };
-  auto stage = [&](uint32_t k0) {
-    float v[32];
-    wreg.values(k0 / 32 + wcc, v);
-    uint32_t h[16], l[16];
+  // units [u, u + S) of the split input (those inside the span; zeros past it): TT blocks a
+  // unit, contiguous, loaded into registers and stored into one of the two LDS buffers
+  constexpr uint32_t STEP = (SPLIT_TOK / SPLIT_N) * SPLIT_BLOCK, P = S * UB / 16, PN = (P + NT - 1) / NT;
+  uint4 sv[PN];
+  auto stage_load = [&](uint32_t u) {
+    const uint32_t nu = u >= u1 ? 0 : u1 - u < S ? u1 - u : S;
+    const QRsrc rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(a.xs + split_block_at(b0, u, kbs)), 0,
+                                                       nu ? (int)((nu - 1) * STEP + UB) : 0, 0x00020000);
 #pragma unroll
-    for (int i = 0; i < 16; i++) split2(v[2 * i], v[2 * i + 1], h[i], l[i]);
-#pragma unroll
-    for (uint32_t g = 0; g < 4; g++) {
-      *(uint4 *)(wt + frag_at(0, wrt, wcc, g, wr)) = make_uint4(h[4 * g], h[4 * g + 1], h[4 * g + 2], h[4 * g + 3]);
-      *(uint4 *)(wt + frag_at(1, wrt, wcc, g, wr)) = make_uint4(l[4 * g], l[4 * g + 1], l[4 * g + 2], l[4 * g + 3]);
+    for (uint32_t k = 0; k < PN; k++) {
+      const uint32_t i = tid + k * NT;
+      sv[k] = qld16(rx, (i / (UB / 16)) * STEP + (i % (UB / 16)) * 16);
     }
   };
-  f32x4 acc[4][4];
+  auto stage_store = [&](uint32_t u) {
+    uint8_t *dst = lds + (((u - u0) / S) & 1) * (S * UB);
 #pragma unroll
-  for (int i = 0; i < 4; i++)
+    for (uint32_t k = 0; k < PN; k++)
+      if ((k + 1) * NT <= P || tid + k * NT < P) *(uint4 *)(dst + (tid + k * NT) * 16) = sv[k];
+  };
+  auto compute = [&](uint32_t d, uint32_t u) {
+    const uint8_t *xl = lds + ((u - u0) % (2 * S)) * UB;
+    // the last unit of a width of 64 (mod 128) columns: its first two blocks
+    const bool half = !W::CHUNK && a.cols - u * QG_U < QG_U;
+    f16x8 w[RT][4], wl[RT][W::LO ? 4 : 1];
+    float dr[RT][W::CHUNK ? 1 : 4], mn[RT];
 #pragma unroll
-    for (int j = 0; j < 4; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  fetch(kb);
-  for (uint32_t k0 = kb; k0 < ke; k0 += QG_K) {
-    bf16x8 Bh[2][4], Bl[2][4];
+    for (uint32_t r = 0; r < RT; r++) buf[d][r].unpack(u, g, w[r], wl[r], dr[r], mn[r]);
 #pragma unroll
-    for (uint32_t ks = 0; ks < 2; ks++)
+    for (uint32_t t = 0; t < TT; t++) {
+      const uint8_t *xb = xl + t * SPLIT_BLOCK;
+      const f32x4 s = *(const f32x4 *)(xb + SPLIT_SCALE + 16 * g);
+      f16x8 xh[4], xo[4];
 #pragma unroll
-      for (uint32_t i = 0; i < 4; i++) {
-        Bh[ks][i] = xfrag(k0, 0, wn * 4 + i, ks);
-        Bl[ks][i] = xfrag(k0, 1, wn * 4 + i, ks);
+      for (uint32_t j = 0; j < 4; j++) {
+        const uint32_t at = W::CHUNK ? (j * 64 + lane) * 16 : ((g * 4 + j) * 16 + c) * 16;
+        xh[j] = *(const f16x8 *)(xb + at);
+        xo[j] = *(const f16x8 *)(xb + at + SPLIT_LO);
       }
-    stage(k0);
-    __syncthreads();
-    if (k0 + QG_K < ke) fetch(k0 + QG_K);  // next tile's loads fly during the MFMAs
+      const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+      if constexpr (W::CHUNK) {
+        f32x4 p[RT];
 #pragma unroll
-    for (uint32_t ks = 0; ks < 2; ks++) {
-      bf16x8 Ah[4], Al[4];
+        for (uint32_t j = 0; j < 4; j++) {
 #pragma unroll
-      for (uint32_t i = 0; i < 4; i++) {
-        Ah[i] = *(const bf16x8 *)(wt + frag_at(0, wm * 4 + i, ks, 0, 0) + 8 * lane);
-        Al[i] = *(const bf16x8 *)(wt + frag_at(1, wm * 4 + i, ks, 0, 0) + 8 * lane);
+          for (uint32_t r = 0; r < RT; r++)
+            p[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh[j], w[r][j], j ? p[r] : zero, 0, 0, 0);
+#pragma unroll
+          for (uint32_t r = 0; r < RT; r++) p[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xo[j], w[r][j], p[r], 0, 0, 0);
+          if constexpr (W::LO) {
+#pragma unroll
+            for (uint32_t r = 0; r < RT; r++) p[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh[j], wl[r][j], p[r], 0, 0, 0);
+          }
+        }
+        if constexpr (W::MIN) {
+          const float xsum = *(const float *)(xb + SPLIT_SUM + 4 * lane);
+#pragma unroll
+          for (uint32_t r = 0; r < RT; r++) acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(xsum, mn[r], acc[r][t], 0, 0, 0);
+        }
+#pragma unroll
+        for (uint32_t r = 0; r < RT; r++)
+#pragma unroll
+          for (int i = 0; i < 4; i++) acc[r][t][i] = fmaf(p[r][i] * dr[r][0], s[i], acc[r][t][i]);
+      } else {
+        f32x4 q[RT];
+#pragma unroll
+        for (uint32_t j = 0; j < 4; j++) {
+          if (half && j >= 2) break;
+          f32x4 p[RT];
+#pragma unroll
+          for (uint32_t r = 0; r < RT; r++) p[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh[j], w[r][j], zero, 0, 0, 0);
+#pragma unroll
+          for (uint32_t r = 0; r < RT; r++) p[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xo[j], w[r][j], p[r], 0, 0, 0);
+#pragma unroll
+          for (uint32_t r = 0; r < RT; r++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) q[r][i] = j ? fmaf(p[r][i], dr[r][j], q[r][i]) : p[r][i] * dr[r][j];
+        }
+#pragma unroll
+        for (uint32_t r = 0; r < RT; r++)
+#pragma unroll
+          for (int i = 0; i < 4; i++) acc[r][t][i] = fmaf(q[r][i], s[i], acc[r][t][i]);
       }
-      // the three products of a tile are 16 MFMAs apart (every tile's first, then second, then third)
-#pragma unroll
-      for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(Bh[ks][j], Ah[i], acc[i][j], 0, 0, 0);
-#pragma unroll
-      for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(Bl[ks][j], Ah[i], acc[i][j], 0, 0, 0);
-#pragma unroll
-      for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(Bh[ks][j], Al[i], acc[i][j], 0, 0, 0);
     }
-    __syncthreads();
+  };
+  stage_load(u0);
+#pragma unroll
+  for (uint32_t d = 0; d < D; d++) fetch(d, u0 + d);
+  stage_store(u0);
+  __syncthreads();
+  for (uint32_t ub = u0; ub < u1; ub += D) {
+#pragma unroll
+    for (uint32_t d = 0; d < D; d++) {
+      const uint32_t u = ub + d;
+      if (d % S == 0) stage_load(u + S);
+      if (u < u1) compute(d, u);
+      fetch(d, u + D);
+      if (d % S == S - 1) {
+        stage_store(u + 1);
+        __syncthreads();
+      }
+    }
   }
-  // The products are formed as X W^T, so lane (g, c) of tile (i, j) holds tokens 16 j + 4 g + e
-  // of row 16 i + c: each store writes 16 consecutive rows of four tokens.
-  const uint32_t row0 = m0 + wm * 64 + (lane & 15);
+  // The products are formed as X W^T, so lane (g, c) of tile (r, t) holds tokens 16 t + 4 g + i
+  // of row 16 r + c: each store writes 16 consecutive rows of four tokens.
+  float *out = a.part ? a.part + (uint64_t)z * a.batch * a.rows_total + jb.row0 : jb.y + jb.row_base;
+  const uint32_t stride = a.part ? a.rows_total : jb.stride;
+  const bool add = a.accumulate && !a.part;  // partials are added by their finish
 #pragma unroll
-  for (int j = 0; j < 4; j++)
+  for (uint32_t r = 0; r < RT; r++) {
+    const uint32_t row = m0 + 16 * r + c;
+    if (row >= jb.rows) continue;
 #pragma unroll
-    for (int e = 0; e < 4; e++) {
-      const uint32_t tok = n0 + wn * 64 + 16 * j + 4 * (lane >> 4) + e;
-      if (tok >= a.batch) continue;
+    for (uint32_t t = 0; t < TT; t++)
 #pragma unroll
       for (int i = 0; i < 4; i++) {
-        const uint32_t row = row0 + 16 * i;
-        if (row >= jb.rows) continue;
-        if (a.part) {
-          a.part[((uint64_t)z * a.batch + tok) * a.rows_total + jb.row0 + row] = acc[i][j][e];
-        } else {
-          float *py = jb.y + (uint64_t)tok * jb.stride + jb.row_base + row;
-          *py = a.accumulate ? *py + acc[i][j][e] : acc[i][j][e];
-        }
+        const uint32_t tok = (b0 + t) * 16 + 4 * g + i;
+        if (tok >= a.batch) continue;
+        float *py = out + (uint64_t)tok * stride + row;
+        *py = add ? *py + acc[r][t][i] : acc[r][t][i];
       }
-    }
+  }
 }
 
 // blockIdx.x walks the jobs' row tiles in order; a job of kind 1 runs the second type.
-template <int T0, int T1>
-__global__ __launch_bounds__(256, 2) void k_gemm_q(QGemm a) {
-  extern __shared__ __attribute__((aligned(16))) uint16_t qlds[];
+template <int T0, int T1, uint32_t TT>
+__global__ __launch_bounds__(qg_threads(TT), 2) void k_gemm_q(QGemm a) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t qlds[];
   uint32_t t = blockIdx.x, j = 0;
   while (j + 1 < a.njobs && t >= a.job[j].tiles) { t -= a.job[j].tiles; j++; }
   const QJob &jb = a.job[j];
-  if (T0 == T1 || jb.kind == 0) gemm_tile<T0>(a, jb, t, qlds);
-  else gemm_tile<T1>(a, jb, t, qlds);
+  if (T0 == T1 || jb.kind == 0) gemm_tile<T0, TT>(a, jb, t, qlds);
+  else gemm_tile<T1, TT>(a, jb, t, qlds);
 }
 
 // Sum of the split-K partials part[z][tok][rows_total] in split order into each job's rows
@@ -539,7 +652,7 @@ __global__ __launch_bounds__(256) void k_gemm_reduce(QGemm a, uint32_t splits) {
 // The GLU finish (k_glu_reduce) of columns k .. k + 7 of token tok.
 template <uint32_t S>
 __device__ __forceinline__ void glu_finish8(const float *part, uint32_t splits, uint32_t R, uint32_t batch, float *y,
-                                            uint16_t *xs, int act, const DeferredNorm &dn, uint32_t tok, uint32_t k) {
+                                            uint8_t *xs, int act, const DeferredNorm &dn, uint32_t tok, uint32_t k) {
   const uint64_t n = (uint64_t)2 * R * batch, row = (uint64_t)tok * 2 * R;
   const __amdgpu_buffer_rsrc_t rp = split_rsrc(part, splits, n);
   const uint32_t sb = (uint32_t)(4 * n), og = (uint32_t)(4 * (row + k)), ou = og + 4 * R;
@@ -576,10 +689,10 @@ __device__ __forceinline__ void glu_finish8(const float *part, uint32_t splits, 
 // consecutive column groups.
 template <uint32_t S>
 __global__ __launch_bounds__(256) void k_glu_reduce(const float *part, uint32_t splits, uint32_t R, uint32_t batch,
-                                                    float *y, uint16_t *xs, int act, DeferredNorm dn, uint32_t by_xcd) {
+                                                    float *y, uint8_t *xs, int act, DeferredNorm dn, uint32_t by_xcd) {
   if (!by_xcd) {
-    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    if (i < batch * (R / 8)) glu_finish8<S>(part, splits, R, batch, y, xs, act, dn, i / (R / 8), (i % (R / 8)) * 8);
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x, c8 = split_kblocks(R) * 16, tok = i / c8, k = (i % c8) * 8;
+    if (tok < batch && k < R) glu_finish8<S>(part, splits, R, batch, y, xs, act, dn, tok, k);
     return;
   }
   const uint32_t x = blockIdx.x % 8, tok = blockIdx.x / 8;
@@ -626,24 +739,29 @@ bool gemm_group_ok(const GemmGroup &g, uint32_t batch) {
   return group_types(g, t) && qgemm_pair(t[0], t[1]);
 }
 
-// K span per workgroup: enough splits for two workgroups per CU, each
-// at least one 256-column block (64 columns when every matrix is Q8_0), and no more partial
-// sums than the scratch holds.
+// 16-token blocks of a workgroup: the smallest of 1, 2, 4 that covers the batch. 65 to 128
+// tokens take two workgroups of 64: with 128 in one, its accumulators leave no registers to load
+// the next activations early (8B prefill in batches of 128: 4.32 against 3.74 ms).
+static uint32_t token_blocks(uint32_t batch) { return batch <= 16 ? 1 : batch <= 32 ? 2 : 4; }
+static uint32_t token_tiles(uint32_t batch) { return (batch + 16 * token_blocks(batch) - 1) / (16 * token_blocks(batch)); }
+
+// K span per workgroup: enough splits for two workgroups per CU, each at least one unit, and
+// no more partial sums than the scratch holds.
 static uint32_t group_kspan(const GemmGroup &g, uint32_t batch, uint64_t scratch_floats, uint32_t *rows_total) {
-  // splits end on K tiles (each chunk reads its own block's header, so a split may start
+  // splits end on units (each chunk reads its own block's header, so a split may start
   // inside a 256-column super-block): finer splits fill the chip closer to its target
-  const uint32_t align = QG_K;
+  const uint32_t align = QG_U;
   uint32_t tiles = 0, rows = 0;
   for (uint32_t j = 0; j < g.n; j++) {
     const Matrix &w = *g.job[j].w;
     tiles += (w.rows + QG_M - 1) / QG_M;
     rows += w.rows;
   }
-  tiles *= (batch + QG_N - 1) / QG_N;
+  tiles *= token_tiles(batch);
   *rows_total = rows;
   const uint32_t cols = g.job[0].w->cols, target = 2 * (uint32_t)device_cu_count();
   uint32_t splits = tiles >= target ? 1 : target / tiles;
-  const uint32_t units = cols / align;
+  const uint32_t units = split_kblocks(cols);
   if (splits > units) splits = units;
   if (splits > 16) splits = 16;
   // The workgroups run in rounds of `target` slots, and a short last round leaves CUs idle
@@ -683,31 +801,40 @@ uint64_t gemm_split_floats(const Matrix &w, uint32_t batch) {
   return gemm_group_split_floats(g, batch);
 }
 
-uint64_t gemm_input_elems(uint32_t cols, uint32_t batch) {
-  return (uint64_t)(batch + QG_N - 1) / QG_N * QG_N * cols * 2;
+uint64_t gemm_input_bytes(uint32_t cols, uint32_t batch) {
+  return (uint64_t)(batch + SPLIT_TOK - 1) / SPLIT_TOK * split_kblocks(cols) * (SPLIT_TOK / SPLIT_N) * SPLIT_BLOCK;
 }
 
 bool gemm_splits_input(const Matrix &w, const GemmScratch *scratch, uint32_t batch) {
-  return qgemm_supported(w) && scratch && scratch->xs && scratch->xs_elems >= gemm_input_elems(w.cols, batch);
+  return qgemm_supported(w) && scratch && scratch->xs && scratch->xs_bytes >= gemm_input_bytes(w.cols, batch);
 }
 
+template <int T0, int T1, uint32_t TT>
+static void launch_qgemm_tt(hipStream_t s, dim3 grid, const QGemm &q) {
+  lds_opt_in((const void *)k_gemm_q<T0, T1, TT>);
+  constexpr uint32_t S = qg_stage(T0, TT) > qg_stage(T1, TT) ? qg_stage(T0, TT) : qg_stage(T1, TT);
+  hipLaunchKernelGGL((k_gemm_q<T0, T1, TT>), grid, dim3(qg_threads(TT)), 2 * S * TT * SPLIT_BLOCK, s, q);
+}
 template <int T0, int T1>
 static void launch_qgemm(hipStream_t s, dim3 grid, const QGemm &q) {
-  lds_opt_in((const void *)k_gemm_q<T0, T1>);
-  hipLaunchKernelGGL((k_gemm_q<T0, T1>), grid, dim3(256), QG_LDS, s, q);
+  switch (token_blocks(q.batch)) {
+    case 1: return launch_qgemm_tt<T0, T1, 1>(s, grid, q);
+    case 2: return launch_qgemm_tt<T0, T1, 2>(s, grid, q);
+    default: return launch_qgemm_tt<T0, T1, 4>(s, grid, q);
+  }
 }
 
 hipError_t gemm_group(hipStream_t s, const GemmGroup &g, const float *x, uint32_t batch, GemmScratch *scratch) {
   if (!batch) return hipSuccess;
   const uint32_t cols = g.job[0].w->cols;
-  if (!gemm_group_ok(g, batch) || !scratch || !scratch->xs || scratch->xs_elems < gemm_input_elems(cols, batch) ||
+  if (!gemm_group_ok(g, batch) || !scratch || !scratch->xs || scratch->xs_bytes < gemm_input_bytes(cols, batch) ||
       (uintptr_t)x % 16)
     return hipErrorInvalidValue;
-  if (g.glu_out && (scratch->xs_elems < gemm_input_elems(g.job[0].w->rows, batch) || (uintptr_t)g.glu_out % 16))
+  if (g.glu_out && (scratch->xs_bytes < gemm_input_bytes(g.job[0].w->rows, batch) || (uintptr_t)g.glu_out % 16))
     return hipErrorInvalidValue;
   if (scratch->xs_of != x || scratch->xs_cols != cols || scratch->xs_batch != batch) {
-    const uint32_t count = (uint32_t)(gemm_input_elems(cols, batch) / 16);
-    hipLaunchKernelGGL(k_gemm_split, dim3((count + 255) / 256), dim3(256), 0, s, x, scratch->xs, cols, batch, count);
+    const uint32_t count = batch * split_kblocks(cols) * 16;
+    hipLaunchKernelGGL(k_gemm_split, dim3((count + 255) / 256), dim3(256), 0, s, x, scratch->xs, cols, count);
     WGD_HIP(hipGetLastError());
     scratch->xs_of = x; scratch->xs_cols = cols; scratch->xs_batch = batch;
   }
@@ -736,7 +863,7 @@ hipError_t gemm_group(hipStream_t s, const GemmGroup &g, const float *x, uint32_
   if (partials && (splits > MAX_SPLITS || (uint64_t)splits * batch * q.rows_total * 4 >= (1ull << 31)))
     return hipErrorInvalidValue;
   q.part = partials ? scratch->p : nullptr;
-  const dim3 grid(tiles, (batch + QG_N - 1) / QG_N, splits);
+  const dim3 grid(tiles, token_tiles(batch), splits);
   const int a = types[0], b = types[1];
   if (a == Q4_K && b == Q4_K) launch_qgemm<Q4_K, Q4_K>(s, grid, q);
   else if (a == Q6_K && b == Q6_K) launch_qgemm<Q6_K, Q6_K>(s, grid, q);
@@ -751,7 +878,7 @@ hipError_t gemm_group(hipStream_t s, const GemmGroup &g, const float *x, uint32_
   else return hipErrorInvalidValue;
   WGD_HIP(hipGetLastError());
   if (g.glu_out) {
-    const uint32_t R = g.job[0].w->rows, count = batch * (R / 8);
+    const uint32_t R = g.job[0].w->rows, count = batch * split_kblocks(R) * 16;
     const uint32_t by_xcd = R % 1024 == 0 && tiles % 8 == 0 ? 1u : 0u;
     const dim3 grid(by_xcd ? batch * 8 : (count + 255) / 256);
     const float *part = q.part;

@@ -75,17 +75,17 @@ hipError_t repack_planar(hipStream_t s, int type, const uint8_t *src, uint8_t *d
 
 // Scratch of the prompt GEMM on planar weights. p: split-K partial sums, of which
 // gemm_split_floats() is what a launch of w over `batch` tokens can use (0: it does not
-// split; less scratch means fewer splits). xs: the activations split into bf16 (hi, lo) in
-// MFMA fragment order, gemm_input_elems() of them (without it the generic kernel runs).
+// split; less scratch means fewer splits). xs: the activations split into f16 (hi, lo) in
+// MFMA fragment order, gemm_input_bytes() of them (without it the generic kernel runs).
 // xs_of/xs_cols/xs_batch name the activations xs holds, so GEMMs over the same input split
 // it once; whoever rewrites that memory clears xs_of.
 struct GemmScratch {
   float *p = nullptr; uint64_t floats = 0;
-  uint16_t *xs = nullptr; uint64_t xs_elems = 0;
+  uint8_t *xs = nullptr; uint64_t xs_bytes = 0;
   const float *xs_of = nullptr; uint32_t xs_cols = 0, xs_batch = 0;
 };
 uint64_t gemm_split_floats(const Matrix &w, uint32_t batch);
-uint64_t gemm_input_elems(uint32_t cols, uint32_t batch);
+uint64_t gemm_input_bytes(uint32_t cols, uint32_t batch);
 // True when a GEMM of w over `batch` tokens runs the planar-weight kernel on the split input
 // (and may add into y).
 bool gemm_splits_input(const Matrix &w, const GemmScratch *scratch, uint32_t batch);
@@ -158,15 +158,15 @@ hipError_t norm(hipStream_t s, const float *x, const float *w, float *y, uint32_
 // split of state * w, and each token's sum of squares of state in residual_split_segs(n)
 // segments to sq, for a consumer that applies the norm factor (DeferredNorm).
 uint32_t residual_split_segs(uint32_t n);
-hipError_t residual_split(hipStream_t s, const float *part, uint32_t splits, float *state, const float *w, uint16_t *xs,
+hipError_t residual_split(hipStream_t s, const float *part, uint32_t splits, float *state, const float *w, uint8_t *xs,
                           float *sq, uint32_t n, uint32_t batch);
 // Per token: state += the split-K partial sums part[z][tok][n] (in split order), then
 // norm_split() of the new state into y and xs (n % 64 == 0, n <= 16384). With post_w the
 // sums are a delta added as RMSNorm(delta) * post_w (Gemma's post-norms).
 hipError_t reduce_norm_split(hipStream_t s, const float *part, uint32_t splits, float *state, const float *w, float *y,
-                             uint16_t *xs, uint32_t n, float eps, uint32_t batch, const float *post_w = nullptr);
+                             uint8_t *xs, uint32_t n, float eps, uint32_t batch, const float *post_w = nullptr);
 // norm() that also writes its output in the prompt GEMM's split form into xs (n % 64 == 0).
-hipError_t norm_split(hipStream_t s, const float *x, const float *w, float *y, uint16_t *xs, uint32_t n, float eps,
+hipError_t norm_split(hipStream_t s, const float *x, const float *w, float *y, uint8_t *xs, uint32_t n, float eps,
                       uint32_t batch);
 // mode 0: Q/K norm + half-split, 1: half-split, 2: adjacent pairs. start_dev overrides start.
 hipError_t rope(hipStream_t s, float *x, const float *w, uint32_t heads, uint32_t hd,
@@ -196,7 +196,7 @@ struct AttnArgs {
   float scale; uint32_t window, capacity, batch;
   float *partial; uint32_t partial_floats;  // split-K scratch (may be null: single split)
   // optional: the output also in the prompt GEMM's split form; *xs_written says whether it was
-  uint16_t *xs = nullptr; bool *xs_written = nullptr;
+  uint8_t *xs = nullptr; bool *xs_written = nullptr;
   bool kv16 = false;
 };
 hipError_t attention(hipStream_t s, const AttnArgs &a);
@@ -207,7 +207,7 @@ uint64_t attention_scratch_floats(uint32_t heads, uint32_t hd, uint32_t batch, u
 hipError_t add(hipStream_t s, const float *delta, float *state, uint32_t n);
 hipError_t glu(hipStream_t s, const float *gate, const float *up, float *y, uint32_t n, int act);
 // glu() over [batch][cols] that also writes y in the prompt GEMM's split form (cols % 64 == 0).
-hipError_t glu_split(hipStream_t s, const float *gate, const float *up, float *y, uint16_t *xs, uint32_t cols,
+hipError_t glu_split(hipStream_t s, const float *gate, const float *up, float *y, uint8_t *xs, uint32_t cols,
                      uint32_t batch, int act);
 hipError_t bias_add(hipStream_t s, float *y, const float *b, uint32_t n, uint32_t width);
 hipError_t activate(hipStream_t s, float *x, uint32_t n);

@@ -26,8 +26,8 @@ struct wgd_context {
   uint64_t mv_qx_bytes = 0;
   float *gemm_part = nullptr;         // split-K partial sums of wgd_matmul's prompt GEMM
   uint64_t gemm_part_floats = 0;
-  uint16_t *gemm_xs = nullptr;        // its input split into bf16 (hi, lo)
-  uint64_t gemm_xs_elems = 0;
+  uint8_t *gemm_xs = nullptr;        // its input split into f16 (hi, lo)
+  uint64_t gemm_xs_bytes = 0;
   wgd::SampleParams *sample_params = nullptr;  // settings of wgd_sample
   void *sample_scratch = nullptr;              // its slices' candidates
   uint64_t sample_scratch_bytes = 0;

@@ -131,7 +131,7 @@ static RopeParams rope_params(wgd_model *m, int l) {
 // Attention of one layer, with RoPE and the KV append unless `prepared` (the Q/K/V GEMM
 // finish did them); positions from start (host) or start_dev.
 hipError_t attention_block(wgd_model *m, int l, uint32_t n, uint32_t start, const int32_t *start_dev,
-                           bool prepared = false, uint16_t *xs = nullptr, bool *xs_written = nullptr) {
+                           bool prepared = false, uint8_t *xs = nullptr, bool *xs_written = nullptr) {
   const wgd_model_config &c = m->c;
   Layer &L = m->L[l];
   hipStream_t s = m->ctx->stream;
@@ -210,7 +210,7 @@ hipError_t layers_batched(wgd_model *m, uint32_t n, uint32_t start, const int32_
   const wgd_model_config &c = m->c;
   hipStream_t s = m->ctx->stream;
   const uint32_t H = c.hidden, qd = c.heads * c.head_dim, kd = c.kv_heads * c.head_dim, F = c.intermediate;
-  // The GEMMs of one input (q, k, v; gate, up) share its bf16 split (xs_of names the buffer
+  // The GEMMs of one input (q, k, v; gate, up) share its f16 split (xs_of names the buffer
   // it was made from and is cleared whenever that buffer is rewritten). RMSNorm and the GLU
   // write the split themselves when the GEMM after them runs on it; the O and down GEMMs
   // then add straight into the residual stream.
@@ -836,14 +836,14 @@ int wgd_model_ready(wgd_model *m) {
       }
   }
   if (rc) return rc;
-  // prompt GEMM scratch: split-K sums and the bf16 split input, the most any layer matrix
+  // prompt GEMM scratch: split-K sums and the f16 split input, the most any layer matrix
   // uses at the batch size
   uint64_t gp = 0, gx = 0;
   for (const Layer &L : m->L) {
     for (const Matrix *w : {&L.q, &L.k, &L.v, &L.o, &L.gate, &L.up, &L.down})
       if (w->data) {
         gp = std::max(gp, gemm_split_floats(*w, (uint32_t)c.batch));
-        gx = std::max(gx, gemm_input_elems(w->cols, (uint32_t)c.batch));
+        gx = std::max(gx, gemm_input_bytes(w->cols, (uint32_t)c.batch));
       }
     gp = std::max(gp, gemm_group_split_floats(qkv_group(m, L), (uint32_t)c.batch));
     if (L.o.data) gp = std::max(gp, gemm_group_split_floats(res_group(m, L.o), (uint32_t)c.batch));
@@ -858,7 +858,7 @@ int wgd_model_ready(wgd_model *m) {
   if (gx && !m->gemm_part.xs) {
     rc = alloc_t(m, gx, "prompt GEMM split input", &m->gemm_part.xs);
     if (rc) return rc;
-    m->gemm_part.xs_elems = gx;
+    m->gemm_part.xs_bytes = gx;
   }
   // a prompt batch's RoPE rotations (the model's theta; Gemma's local theta too)
   if (!m->rope_batch[0]) {

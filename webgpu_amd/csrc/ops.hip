@@ -44,7 +44,7 @@ hipError_t norm(hipStream_t s, const float *x, const float *w, float *y, uint32_
 
 // One token per workgroup, eight consecutive elements per thread step: the f32 output and
 // its split form for the GEMMs that read it.
-__global__ __launch_bounds__(256) void k_norm_split(const float *x, const float *w, float *y, uint16_t *xs,
+__global__ __launch_bounds__(256) void k_norm_split(const float *x, const float *w, float *y, uint8_t *xs,
                                                     uint32_t n, float eps) {
   __shared__ float red[4];
   const uint32_t tok = blockIdx.x;
@@ -88,7 +88,7 @@ __device__ __forceinline__ float block_total(float ss, float *red) {
 }
 __global__ __launch_bounds__(512) void k_reduce_norm_split(const float *part, uint32_t splits, float *state,
                                                            const float *post_w, const float *w, float *y,
-                                                           uint16_t *xs, uint32_t n, uint32_t batch, float eps) {
+                                                           uint8_t *xs, uint32_t n, uint32_t batch, float eps) {
   __shared__ float red[RN_T / 64];
   const uint32_t tok = blockIdx.x, tid = threadIdx.x;
   const uint64_t stride = (uint64_t)n * batch;
@@ -163,7 +163,7 @@ constexpr uint32_t RS_T = 128, RS_E = 8 * RS_T;
 static bool residual_by_xcd(uint32_t n) { return n % 1024 == 0; }
 uint32_t residual_split_segs(uint32_t n) { return residual_by_xcd(n) ? 8 : (n + RS_E - 1) / RS_E; }
 __global__ __launch_bounds__(128) void k_residual_split(const float *part, uint32_t splits, float *state,
-                                                        const float *w, uint16_t *xs, float *sq, uint32_t n,
+                                                        const float *w, uint8_t *xs, float *sq, uint32_t n,
                                                         uint32_t batch, uint32_t by_xcd) {
   __shared__ float red[RS_T / 64];
   const uint32_t seg = blockIdx.x, tok = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
@@ -195,10 +195,10 @@ __global__ __launch_bounds__(128) void k_residual_split(const float *part, uint3
   if (tid == 0) sq[(uint64_t)tok * gridDim.x + seg] = red[0] + red[1];
 }
 
-hipError_t residual_split(hipStream_t s, const float *part, uint32_t splits, float *state, const float *w, uint16_t *xs,
+hipError_t residual_split(hipStream_t s, const float *part, uint32_t splits, float *state, const float *w, uint8_t *xs,
                           float *sq, uint32_t n, uint32_t batch) {
   if (!batch) return hipSuccess;
-  if (n % SPLIT_K || !splits || splits > MAX_SPLITS || (uint64_t)splits * n * batch * 4 >= (1ull << 31) || !sq ||
+  if (n % SPLIT_COLS || !splits || splits > MAX_SPLITS || (uint64_t)splits * n * batch * 4 >= (1ull << 31) || !sq ||
       ((uintptr_t)part | (uintptr_t)state | (uintptr_t)w) % 16)
     return hipErrorInvalidValue;
   hipLaunchKernelGGL(k_residual_split, dim3(residual_split_segs(n), batch), dim3(RS_T), 0, s, part, splits, state, w,
@@ -207,9 +207,9 @@ hipError_t residual_split(hipStream_t s, const float *part, uint32_t splits, flo
 }
 
 hipError_t reduce_norm_split(hipStream_t s, const float *part, uint32_t splits, float *state, const float *w, float *y,
-                             uint16_t *xs, uint32_t n, float eps, uint32_t batch, const float *post_w) {
+                             uint8_t *xs, uint32_t n, float eps, uint32_t batch, const float *post_w) {
   if (!batch) return hipSuccess;
-  if (n % SPLIT_K || n > RN_G * 8 * RN_T || !splits || splits > MAX_SPLITS ||
+  if (n % SPLIT_COLS || n > RN_G * 8 * RN_T || !splits || splits > MAX_SPLITS ||
       (uint64_t)splits * n * batch * 4 >= (1ull << 31) ||
       ((uintptr_t)part | (uintptr_t)state | (uintptr_t)w | (uintptr_t)y | (uintptr_t)post_w) % 16)
     return hipErrorInvalidValue;
@@ -218,10 +218,10 @@ hipError_t reduce_norm_split(hipStream_t s, const float *part, uint32_t splits, 
   return hipGetLastError();
 }
 
-hipError_t norm_split(hipStream_t s, const float *x, const float *w, float *y, uint16_t *xs, uint32_t n, float eps,
+hipError_t norm_split(hipStream_t s, const float *x, const float *w, float *y, uint8_t *xs, uint32_t n, float eps,
                       uint32_t batch) {
   if (!batch) return hipSuccess;
-  if (n % SPLIT_K || ((uintptr_t)x | (uintptr_t)w | (uintptr_t)y) % 16) return hipErrorInvalidValue;
+  if (n % SPLIT_COLS || ((uintptr_t)x | (uintptr_t)w | (uintptr_t)y) % 16) return hipErrorInvalidValue;
   hipLaunchKernelGGL(k_norm_split, dim3(batch), dim3(256), 0, s, x, w, y, xs, n, eps);
   return hipGetLastError();
 }
@@ -524,12 +524,11 @@ hipError_t glu(hipStream_t s, const float *gate, const float *up, float *y, uint
   return hipGetLastError();
 }
 
-// Eight consecutive elements of one token per thread.
-__global__ __launch_bounds__(256) void k_glu_split(const float *g, const float *u, float *y, uint16_t *xs,
+// Eight consecutive elements of one token per thread, 16 threads per 128 columns.
+__global__ __launch_bounds__(256) void k_glu_split(const float *g, const float *u, float *y, uint8_t *xs,
                                                    uint32_t cols, uint32_t count, int act) {
-  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= count) return;
-  const uint32_t c8 = cols / 8, tok = i / c8, k = (i % c8) * 8;
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x, c8 = split_kblocks(cols) * 16, tok = i / c8, k = (i % c8) * 8;
+  if (i >= count || k >= cols) return;
   const uint64_t o = (uint64_t)tok * cols + k;
   float v[8];
 #pragma unroll
@@ -548,11 +547,11 @@ __global__ __launch_bounds__(256) void k_glu_split(const float *g, const float *
   split_store8(xs, cols, tok, k, a, b);
 }
 
-hipError_t glu_split(hipStream_t s, const float *gate, const float *up, float *y, uint16_t *xs, uint32_t cols,
+hipError_t glu_split(hipStream_t s, const float *gate, const float *up, float *y, uint8_t *xs, uint32_t cols,
                      uint32_t batch, int act) {
   if (!batch) return hipSuccess;
-  if (cols % SPLIT_K || ((uintptr_t)gate | (uintptr_t)up | (uintptr_t)y) % 16) return hipErrorInvalidValue;
-  const uint32_t count = batch * (cols / 8);
+  if (cols % SPLIT_COLS || ((uintptr_t)gate | (uintptr_t)up | (uintptr_t)y) % 16) return hipErrorInvalidValue;
+  const uint32_t count = batch * split_kblocks(cols) * 16;
   hipLaunchKernelGGL(k_glu_split, dim3((count + 255) / 256), dim3(256), 0, s, gate, up, y, xs, cols, count, act);
   return hipGetLastError();
 }
