@@ -253,6 +253,34 @@ def test_attention_long_context_and_ring(gpu, context, start, batch, window, cap
         gpu.destroy(b)
 
 
+# The row-slice kernel (head_dim 64 / 128) at its edges: one query, tiles of
+# 16 ragged and whole, groups that leave wavefronts idle (3) or take two workgroups (12), key
+# slices that are empty, rings shorter than a block of 16 and rings wrapped inside a block, a window
+# that starts inside a block, 16 key splits, and a ninth query tile of one query. The bound is f32's:
+# sums of up to 3100 keys and 128 products, about 2^-24 * sqrt(keys) of values of order one, with margin.
+@pytest.mark.parametrize("heads,kvh,hd,start,batch,window,capacity", [
+    (4, 1, 128, 0, 1, 4096, 64), (3, 1, 64, 5, 2, 4096, 7), (12, 1, 128, 30, 17, 9, 25), (8, 8, 64, 15, 16, 4096, 31),
+    (2, 1, 128, 3000, 16, 4096, 3016), (16, 2, 64, 333, 33, 100, 140), (6, 2, 128, 250, 128, 4096, 400),
+    (16, 1, 64, 40, 128, 64, 191), (4, 2, 128, 11, 129, 4096, 256), (32, 8, 128, 240, 10, 4096, 256)])
+@pytest.mark.parametrize("half", [False, True])
+def test_attention_row_slices(gpu, heads, kvh, hd, start, batch, window, capacity, half):
+    rng = np.random.default_rng(heads * hd + start + batch)
+    q = rng.standard_normal(batch * heads * hd).astype(np.float32)
+    k, v = (rng.standard_normal(capacity * kvh * hd).astype(np.float16 if half else np.float32) for _ in range(2))
+    if start + batch < capacity:  # slots past the keys are never read into a result
+        k[(start + batch) * kvh * hd:] = np.nan
+        v[(start + batch) * kvh * hd:] = np.nan
+    bufs = [gpu.upload(a, nm) for a, nm in ((q, "q"), (k, "k"), (v, "v"))] + [gpu.buffer(q.nbytes, "y")]
+    scale = float(1 / np.sqrt(hd))
+    run = gpu.attention_f16kv if half else gpu.attention
+    run(*bufs, heads, kvh, hd, start, scale, window, capacity, capacity, batch)
+    got = gpu.read_f32(bufs[3], q.size)
+    want = orc.attention(q, k.astype(np.float64), v.astype(np.float64), heads, kvh, hd, start, scale, window, capacity, batch)
+    near(got, want, 2e-5, "row slices")
+    for b in bufs:
+        gpu.destroy(b)
+
+
 # Prompt batches (the matrix-core path for head_dim 64/128/256): causal from position 0,
 # a batch deep in the context, a ragged batch with one query head per KV head, a sliding
 # window shorter than the batch's key range, and a wrapped ring. The last two split the

@@ -241,8 +241,8 @@ static void launch_attention_combine(hipStream_t s, const float *part, float *y,
     hipLaunchKernelGGL(k_attention_combine, dim3(rows), dim3(128), 0, s, part, y, rows, hd, nsplit, xs, heads);
 }
 
-// Prompt batches on the f32 matrix cores (v_mfma_f32_16x16x4_f32: f32 products, f32 sums, as
-// the f32 shader computes them). A wavefront owns 16 consecutive queries of one head; the
+// Prompt batches at head dim 256 on the f32 matrix cores (v_mfma_f32_16x16x4_f32: f32 products,
+// f32 sums, as the f32 shader computes them). A wavefront owns 16 consecutive queries of one head; the
 // four wavefronts of a workgroup share one kv head and stage 64-key tiles of K (row-major)
 // and V (transposed) in LDS. Scores are formed transposed, S^T = K Q^T, so lane (g, c) holds
 // keys 4g..4g+3 of query row c: a row's running max and sum live in its own lanes (two
@@ -405,6 +405,189 @@ static hipError_t launch_attn_prompt(hipStream_t s, AttnK a, const AttnArgs &in,
   return hipSuccess;
 }
 
+// Prompt batches at head dims 64 and 128. k_attn_prompt stages 64-key tiles of K and V through
+// LDS for four (head, query tile) rows, with two barriers and a chain of 256 f32 MFMAs (4096
+// cycles) per tile and few wavefronts where the batch is small. Here each wavefront owns one
+// head's 16 queries and a slice of the keys, reads K and V straight into the MFMA operands (the
+// heads of a kv head share the lines in their CU's cache) and meets no barrier until the slices of
+// its workgroup merge in LDS; a launch of one key split writes the finished output and its
+// split form. Against k_attn_prompt at these head dims (us, merge included):
+//   32 heads, 16 kv heads, 8191 keys, 16 queries, f32: 99 -> 47 (134 MB of K and V: 2.8 TB/s)
+//   32 / 8 heads, 4000 keys, 32 queries: 65 -> 42; 128 queries, f16: 131 -> 113
+//   16 / 16 heads, 2000 keys, 128 queries: 53 -> 43; 256 queries: 80 -> 70
+//   16 / 8 heads, 64 keys, 64 queries: 15.1 -> 12.4; 2 / 2 heads, 9000 keys, 20 queries: 134 -> 27
+// and no slower at any shape tried (32 / 8 heads, 2000 keys, 512 queries: 232 -> 229). The f32
+// MFMAs bound the long ones: 64 per 16 keys, query tile and head, 2048 cycles.
+// One slice holds whole 16-key blocks:
+//   S^T = K Q^T: lane (g, c) loads 16-byte pieces d = 16 t + 4 g of key c, and holds the
+//     scores of keys 4 g .. + 4 for query c, so a query's maximum and sum live in its lanes;
+//   O^T += V^T P^T: MFMA i sums over the keys 4 g + i, whose probabilities lane (g, c) holds
+//     already; it loads d = 64 h + 4 c of key 4 g + i, and output tile (h, e) is the
+//     dimensions 64 h + 4 m + e, so lane (g, c) ends with 16 consecutive ones of query c.
+// f32 products and sums, as in k_attn_prompt.
+template <uint32_t HD, class E>
+__global__ __launch_bounds__(512) void k_attn_rows(AttnK a, uint32_t hp, uint32_t sl, uint8_t *xs) {
+  constexpr uint32_t NT = HD / 16, NH = HD / 64, OS = HD + 4, WS = 32 + 16 * OS;
+  extern __shared__ float lds[];
+  const uint32_t tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c = lane & 15;
+  const uint32_t w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t kv = blockIdx.x, z = blockIdx.z, hgs = (a.group + hp - 1) / hp;
+  const uint32_t qt = blockIdx.y / hgs, h0 = blockIdx.y % hgs * hp;  // first head of the workgroup in its kv head
+  const uint32_t s0 = a.start_dev ? (uint32_t)*a.start_dev : a.start;
+  // the query tile's keys, in blocks of 16, and this wavefront's slice of them
+  const uint32_t first_end = s0 + qt * 16 + 1, last_end = s0 + min(a.batch, qt * 16 + 16);
+  const uint32_t begin0 = first_end - min(first_end, a.window);
+  const uint32_t blocks = (last_end - begin0 + 15) / 16, slices = sl * a.nsplit, per = (blocks + slices - 1) / slices;
+  const uint32_t lo = begin0 + 16 * per * (z * sl + w / hp), hi = min(lo + 16 * per, last_end);
+  const uint32_t hw = h0 + w % hp, h = kv * a.group + hw;
+  const uint32_t b = qt * 16 + c;
+  const bool row_ok = hw < a.group && b < a.batch;
+  const uint32_t end_b = s0 + b + 1, begin_b = end_b - min(end_b, a.window);
+  const uint32_t cap = a.capacity;
+  auto slot = [&](uint32_t base, uint32_t off) {  // (base + off) % cap for base < cap, off < 16
+    const uint32_t s = base + off;
+    return cap >= 16 ? (s >= cap ? s - cap : s) : s % cap;
+  };
+  f32x4 o[NH][4];
+#pragma unroll
+  for (uint32_t x = 0; x < NH; x++)
+#pragma unroll
+    for (uint32_t e = 0; e < 4; e++) o[x][e] = f32x4{0, 0, 0, 0};
+  float m = -INFINITY, l = 0.f;
+  if (hw < a.group && lo < hi) {  // wavefront-uniform
+    f32x4 qr[NT], kr[NT];
+#pragma unroll
+    for (uint32_t t = 0; t < NT; t++)
+      qr[t] = row_ok ? *(const f32x4 *)(a.q + ((uint64_t)b * a.heads + h) * HD + 16 * t + 4 * g) : f32x4{0, 0, 0, 0};
+    auto load_k = [&](uint32_t base) {
+      const uint64_t at = ((uint64_t)slot(base, c) * a.kvh + kv) * HD + 4 * g;
+#pragma unroll
+      for (uint32_t t = 0; t < NT; t++) {
+        const float4 v = kv_get4<E>(a.k, at + 16 * t);
+        kr[t] = f32x4{v.x, v.y, v.z, v.w};
+      }
+    };
+    uint32_t base = lo % cap;
+    load_k(base);
+    for (uint32_t t0 = lo; t0 < hi; t0 += 16) {
+      float4 vr[4][NH];
+#pragma unroll
+      for (uint32_t i = 0; i < 4; i++) {
+        const uint64_t at = ((uint64_t)slot(base, 4 * g + i) * a.kvh + kv) * HD + 4 * c;
+#pragma unroll
+        for (uint32_t x = 0; x < NH; x++) vr[i][x] = kv_get4<E>(a.v, at + 64 * x);
+      }
+      f32x4 a0 = {0, 0, 0, 0}, a1 = {0, 0, 0, 0};  // two chains of MFMAs
+#pragma unroll
+      for (uint32_t t = 0; t < NT; t += 2) {
+#pragma unroll
+        for (uint32_t u = 0; u < 4; u++) {
+          a0 = __builtin_amdgcn_mfma_f32_16x16x4f32(kr[t][u], qr[t][u], a0, 0, 0, 0);
+          a1 = __builtin_amdgcn_mfma_f32_16x16x4f32(kr[t + 1][u], qr[t + 1][u], a1, 0, 0, 0);
+        }
+      }
+      base = slot(base, 15);
+      base = slot(base, 1);
+      if (t0 + 16 < hi) load_k(base);
+      float s[4], mx = -INFINITY;
+#pragma unroll
+      for (uint32_t i = 0; i < 4; i++) {
+        const uint32_t key = t0 + 4 * g + i;
+        s[i] = row_ok && key >= begin_b && key < end_b && key < hi ? (a0[i] + a1[i]) * a.scale : -INFINITY;
+        mx = fmaxf(mx, s[i]);
+      }
+      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      const float mn = fmaxf(m, mx);
+      const float corr = mn == -INFINITY ? 1.f : expf(m - mn);
+      float sum = 0.f;
+#pragma unroll
+      for (uint32_t i = 0; i < 4; i++) {
+        s[i] = s[i] == -INFINITY ? 0.f : expf(s[i] - mn);
+        sum += s[i];
+      }
+      sum += __shfl_xor(sum, 16, 64);
+      sum += __shfl_xor(sum, 32, 64);
+      l = l * corr + sum;
+      m = mn;
+      if (t0 + 16 > hi) {  // slots past the keys hold anything
+#pragma unroll
+        for (uint32_t i = 0; i < 4; i++)
+          if (t0 + 4 * g + i >= hi)
+#pragma unroll
+            for (uint32_t x = 0; x < NH; x++) vr[i][x] = make_float4(0.f, 0.f, 0.f, 0.f);
+      }
+#pragma unroll
+      for (uint32_t x = 0; x < NH; x++)
+#pragma unroll
+        for (uint32_t e = 0; e < 4; e++) o[x][e] *= corr;
+#pragma unroll
+      for (uint32_t i = 0; i < 4; i++)
+#pragma unroll
+        for (uint32_t x = 0; x < NH; x++) {
+          o[x][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(vr[i][x].x, s[i], o[x][0], 0, 0, 0);
+          o[x][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(vr[i][x].y, s[i], o[x][1], 0, 0, 0);
+          o[x][2] = __builtin_amdgcn_mfma_f32_16x16x4f32(vr[i][x].z, s[i], o[x][2], 0, 0, 0);
+          o[x][3] = __builtin_amdgcn_mfma_f32_16x16x4f32(vr[i][x].w, s[i], o[x][3], 0, 0, 0);
+        }
+    }
+  }
+  // lane (g, c): o[x][e][r] is dimension 64 x + 16 g + 4 r + e of query c
+  float *mine = lds + w * WS;
+  if (g == 0) { mine[2 * c] = m; mine[2 * c + 1] = l; }
+#pragma unroll
+  for (uint32_t x = 0; x < NH; x++)
+#pragma unroll
+    for (uint32_t r = 0; r < 4; r++)
+      *(f32x4 *)(mine + 32 + c * OS + 64 * x + 16 * g + 4 * r) = f32x4{o[x][0][r], o[x][1][r], o[x][2][r], o[x][3][r]};
+  __syncthreads();
+  // the slices in order; eight dimensions of a row per thread
+  for (uint32_t i = tid; i < hp * 2 * HD; i += blockDim.x) {
+    const uint32_t d = i % (HD / 8) * 8, qi = i / (HD / 8) % 16, hh = i / (2 * HD), tok = qt * 16 + qi;
+    if (tok >= a.batch || h0 + hh >= a.group) continue;
+    float M = -INFINITY, L = 0.f, v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    for (uint32_t u = 0; u < sl; u++) M = fmaxf(M, lds[(u * hp + hh) * WS + 2 * qi]);
+    for (uint32_t u = 0; u < sl; u++) {
+      const float *p = lds + (u * hp + hh) * WS;
+      if (p[2 * qi] == -INFINITY) continue;
+      const float f = expf(p[2 * qi] - M);
+      L += p[2 * qi + 1] * f;
+      const f32x4 x0 = *(const f32x4 *)(p + 32 + qi * OS + d), x1 = *(const f32x4 *)(p + 32 + qi * OS + d + 4);
+#pragma unroll
+      for (int e = 0; e < 4; e++) { v[e] += x0[e] * f; v[4 + e] += x1[e] * f; }
+    }
+    const uint32_t head = kv * a.group + h0 + hh;
+    const uint64_t row = (uint64_t)tok * a.heads + head;
+    if (a.nsplit == 1) {
+      const float inv = L > 0.f ? 1.f / L : 0.f;
+      const float4 ya = make_float4(v[0] * inv, v[1] * inv, v[2] * inv, v[3] * inv);
+      const float4 yb = make_float4(v[4] * inv, v[5] * inv, v[6] * inv, v[7] * inv);
+      *(float4 *)(a.y + row * HD + d) = ya;
+      *(float4 *)(a.y + row * HD + d + 4) = yb;
+      if (HD % SPLIT_K == 0 && xs) split_store8(xs, a.heads * HD, tok, head * HD + d, ya, yb);
+    } else {
+      float *pp = a.part + ((uint64_t)z * a.batch * a.heads + row) * (HD + 2);
+      if (d == 0) { pp[0] = M; pp[1] = L; }
+#pragma unroll
+      for (int e = 0; e < 8; e++) pp[2 + d + e] = v[e];
+    }
+  }
+}
+
+template <uint32_t HD, class E>
+static hipError_t launch_attn_rows(hipStream_t s, AttnK a, const AttnArgs &in, uint32_t nsplit) {
+  const uint32_t nqt = (in.batch + 15) / 16, hp = a.group < 8 ? a.group : 8, sl = 8 / hp;
+  uint8_t *xs = in.xs && in.hd % SPLIT_K == 0 ? in.xs : nullptr;
+  a.nsplit = nsplit;
+  lds_opt_in((const void *)k_attn_rows<HD, E>);
+  hipLaunchKernelGGL((k_attn_rows<HD, E>), dim3(in.kv_heads, nqt * ((a.group + hp - 1) / hp), nsplit), dim3(64 * hp * sl),
+                     (32 + 16 * (HD + 4)) * sizeof(float) * hp * sl, s, a, hp, sl, xs);
+  WGD_HIP(hipGetLastError());
+  if (nsplit > 1) launch_attention_combine(s, (const float *)in.partial, in.y, in.batch * in.heads, in.hd, nsplit, xs, in.heads);
+  if (in.xs_written) *in.xs_written = xs != nullptr;
+  return hipGetLastError();
+}
+
 static uint32_t tile_keys(uint32_t hd) {
   uint32_t t = 4096 / hd;
   if (t > 64) t = 64;
@@ -416,10 +599,11 @@ uint64_t attention_scratch_floats(uint32_t heads, uint32_t hd, uint32_t batch, u
   return (uint64_t)max_splits * batch * heads * (hd + 2);
 }
 
-// How a launch runs: the MFMA prompt kernel (hd 64/128/256 with 16-byte aligned operands) or
+// How a launch runs: the MFMA kernels (k_attn_rows at hd 64/128, k_attn_prompt at 256, with
+// 16-byte aligned operands) or
 // the generic one (query blocks of qb tokens, tiles of T keys), and the number of key
 // chunks: as many as fill the chip, fewer when `partial_floats` holds fewer partials.
-struct AttnPlan { uint32_t mfma_hd, nsplit, qb, R, T, qblocks; };
+struct AttnPlan { uint32_t mfma_hd, rows, nsplit, qb, R, T, qblocks; };
 static bool attn_plan(const AttnArgs &in, uint64_t partial_floats, AttnPlan &p) {
   const uint32_t group = in.heads / in.kv_heads;
   // Key range bound: the host start when known, else the whole ring/window.
@@ -438,9 +622,22 @@ static bool attn_plan(const AttnArgs &in, uint64_t partial_floats, AttnPlan &p) 
   if (aligned && (in.hd == 64 || in.hd == 128 || in.hd == 256)) {
     p.mfma_hd = in.hd;
     const uint32_t nqt = (in.batch + 15) / 16;
-    const uint32_t wgs = in.kv_heads * ((nqt * group + 3) / 4);
-    tiles = (keys + AP_T - 1) / AP_T;
-    want = ((uint32_t)device_cu_count() * 2 + wgs - 1) / wgs;  // two workgroups per CU: a second wavefront per SIMD
+    p.rows = in.hd <= 128;  // at 256, k_attn_rows' operands would not fit its registers
+    if (p.rows) {
+      const uint32_t hp = group < 8 ? group : 8, sl = 8 / hp, wgs = in.kv_heads * nqt * ((group + hp - 1) / hp);
+      // a block of 16 keys per wavefront at least (two, in fewer splits: 8B prompt in 16s 6.00
+      // -> 6.16 ms), and eight wavefronts per CU (at hd 64, whose wavefronts hold half as much in
+      // flight, 16: 128 heads over 6000 keys, 128 queries, 354 -> 328 us), at most the 16 splits that
+      // the merge loads at once. Rounded down, so the partials never outgrow 16 * 8 rows per
+      // workgroup in flight.
+      tiles = ((keys + 15) / 16 + sl - 1) / sl;
+      want = (uint32_t)device_cu_count() * (in.hd == 64 ? 2 : 1) / wgs;
+      if (want > 16) want = 16;
+    } else {
+      const uint32_t wgs = in.kv_heads * ((nqt * group + 3) / 4);
+      tiles = (keys + AP_T - 1) / AP_T;
+      want = ((uint32_t)device_cu_count() * 2 + wgs - 1) / wgs;  // two workgroups per CU: a second wavefront per SIMD
+    }
   } else {
     p.qb = group >= 16 ? 1 : 16 / group;
     if (p.qb > in.batch) p.qb = in.batch;
@@ -479,8 +676,8 @@ hipError_t attention(hipStream_t s, const AttnArgs &in) {
   a.group = in.heads / in.kv_heads;
   AttnPlan p;
   if (!attn_plan(in, in.partial ? in.partial_floats : 0, p)) return hipErrorInvalidValue;
-  if (p.mfma_hd == 64) return in.kv16 ? launch_attn_prompt<64, _Float16>(s, a, in, p.nsplit) : launch_attn_prompt<64, float>(s, a, in, p.nsplit);
-  if (p.mfma_hd == 128) return in.kv16 ? launch_attn_prompt<128, _Float16>(s, a, in, p.nsplit) : launch_attn_prompt<128, float>(s, a, in, p.nsplit);
+  if (p.rows && in.hd == 64) return in.kv16 ? launch_attn_rows<64, _Float16>(s, a, in, p.nsplit) : launch_attn_rows<64, float>(s, a, in, p.nsplit);
+  if (p.rows) return in.kv16 ? launch_attn_rows<128, _Float16>(s, a, in, p.nsplit) : launch_attn_rows<128, float>(s, a, in, p.nsplit);
   if (p.mfma_hd == 256) return in.kv16 ? launch_attn_prompt<256, _Float16>(s, a, in, p.nsplit) : launch_attn_prompt<256, float>(s, a, in, p.nsplit);
   a.qb = p.qb; a.R = p.R; a.T = p.T;
   const uint32_t qblocks = p.qblocks, nsplit = p.nsplit;
