@@ -30,6 +30,20 @@ def _cases():
     l[rng.integers(0, 3000, 20)] = -np.inf
     yield "non-finite", l, 0.5, 10, 0.8
     yield "signed-zeros", np.array([0.0, -0.0, -1.0, 0.0, -0.0, -3.0], np.float32), 2.0, 4, 1.0
+    # the bound from the slices' best logits: as many slices as k and one fewer, a slice that holds
+    # more than 64 of the largest, slices without a finite logit, and one slice holding so many
+    # that the histogram takes over
+    yield "k-is-slices", rng.standard_normal(40 * 1024).astype(np.float32), 0.9, 40, 0.95
+    yield "k-over-slices", rng.standard_normal(39 * 1024 + 5).astype(np.float32), 0.9, 40, 0.95
+    l = rng.standard_normal(100000).astype(np.float32)
+    l[2000:2150] += 9
+    yield "one-rich-slice", l, 2.0, 90, 1.0
+    l = np.full(150000, np.nan, np.float32)
+    l[70000:75000] = rng.standard_normal(5000)
+    yield "empty-slices", l, 1.5, 50, 0.99
+    l = rng.standard_normal(200000).astype(np.float32)
+    l[5000:9000] = 8
+    yield "ties-fill-slices", l, 1.0, 150, 1.0
     yield "one", np.array([-5.0], np.float32), 0.7, 40, 0.9
     yield "fewer-than-k", np.array([1.0, np.nan, 2.0, 2.0, -1.0, np.inf, 0.5], np.float32), 1.2, 40, 0.9
 

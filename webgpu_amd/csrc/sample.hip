@@ -20,11 +20,18 @@
 //     histogram of the top 12 key bits, and every composite at or above the bin holding the
 //     slice's k-th largest. That is a superset of the slice's top k, so together the slices
 //     hold the row's top k.
-//   * k_sample, one workgroup of 1024 threads over those candidates: a 4096-bin histogram of
-//     the top 12 composite bits and a block scan find the bin holding the k-th largest; if it
-//     and the bins above hold at most 1024 candidates they are gathered into LDS, otherwise
-//     the next 12 bits of that bin are histogrammed (values that tie over many indices) until
-//     they fit. Each gathered composite's rank orders them; then the probabilities and draw.
+//   * k_sample, one workgroup of 1024 threads over those candidates. With at least k slices, the
+//     k-th largest of the slices' best composites is a lower bound of the row's k-th
+//     largest (k composites reach it), and few candidates lie above it: they are gathered
+//     into LDS at once (each wavefront reads its slices' lists, the first 64 entries loaded
+//     before the bound is known). Otherwise, or if more than 1024 lie above it, a 4096-bin
+//     histogram of the top 12 composite bits and a block scan find the bin holding the k-th
+//     largest; if it and the bins above hold at most 1024 candidates they are gathered into
+//     LDS, else the next 12 bits of that bin are histogrammed (values that tie over many
+//     indices) until they fit. Each gathered composite's rank orders them; then the
+//     probabilities, their running sum (one thread, in order) and the draw.
+//     It is a chain of latencies in one workgroup, not of bytes: 128256 logits, k = 40, took
+//     19.9 us by the histogram and serial sums with a division per step, 12.1 us so.
 #include "internal.h"
 #include "decode.h"
 
@@ -50,6 +57,11 @@ __device__ __forceinline__ uint32_t order_key(float v) {
 }
 __device__ __forceinline__ bool finite_f(float v) { return (__float_as_uint(v) & 0x7F800000u) != 0x7F800000u; }
 __device__ __forceinline__ uint32_t comp_index(uint64_t c) { return 0xFFFFFFFFu - (uint32_t)c; }
+// The logit of a composite (order_key undone; -0 comes back as +0).
+__device__ __forceinline__ float comp_value(uint64_t c) {
+  const uint32_t k = (uint32_t)(c >> 32);
+  return __uint_as_float((k & 0x80000000u) ? k & 0x7FFFFFFFu : ~k);
+}
 
 __device__ __forceinline__ uint32_t wave_sum_u32(uint32_t v) {
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
@@ -172,38 +184,28 @@ __global__ __launch_bounds__(SL_T) void k_sample_local(const float *logits, uint
 struct SampleLds {
   uint32_t hist[SMP_BINS];
   uint64_t cand[SMP_CAND];
-  double prob[256];
+  double prob[256], cum[256];
+  uint64_t top[SL_MAX];
+  uint32_t counts[SL_MAX];
   uint32_t offs[SL_MAX + 1];
   uint32_t wsum[16];
   uint64_t wmax[16];
-  uint32_t bin, above, ncand;
+  uint64_t bound;
+  uint32_t bin, above, ncand, cutoff;
 };
 
-// The token from the slices' candidates; st (optional) receives it as k_argmax_advance would.
-__global__ __launch_bounds__(SMP_T) void k_sample(const float *logits, const uint64_t *cand, const SliceOut *so,
-                                                  uint32_t nslices, uint32_t slice, const SampleParams *prm,
-                                                  int32_t index, StepState *st, int32_t *out, int32_t *tokens,
-                                                  uint32_t cap, int advance) {
-  __shared__ SampleLds L;
-  const uint32_t tid = threadIdx.x, lane = tid & 63;
-  const SampleParams p = *prm;
-  // the slices' totals, and the offsets of their candidate lists in one flat range [0, C):
-  // one summary per thread (all loads at once), then a scan by thread 0 in LDS
-  const SliceOut mine_so = tid < nslices ? so[tid] : SliceOut{0, 0, 0};
-  if (tid < nslices) L.offs[tid + 1] = mine_so.count;
-  uint32_t cnt = wave_sum_u32(mine_so.finite);
-  uint64_t best = wave_max_u64(mine_so.best);
-  if (lane == 0) { L.wsum[tid >> 6] = cnt; L.wmax[tid >> 6] = best; }
-  __syncthreads();
+// The histogram selection of k_sample: the candidates at or above a bin's start that hold the
+// K largest, through put().
+template <class Put>
+__device__ __forceinline__ void select(SampleLds &L, const uint64_t *cand, uint32_t slice, uint32_t nslices, uint32_t K,
+                                       Put put) {
+  const uint32_t tid = threadIdx.x;
+  // the offsets of the slices' candidate lists in one flat range [0, C)
   if (tid == 0) {
     L.offs[0] = 0;
-    for (uint32_t w = 0; w < nslices; w++) L.offs[w + 1] += L.offs[w];
+    for (uint32_t w = 0; w < nslices; w++) L.offs[w + 1] = L.offs[w] + L.counts[w];
   }
-  cnt = 0; best = 0;
-  for (uint32_t u = 0; u < SMP_T / 64; u++) {
-    cnt += L.wsum[u];
-    best = L.wmax[u] > best ? L.wmax[u] : best;
-  }
+  for (uint32_t b = tid; b < SMP_BINS; b += SMP_T) L.hist[b] = 0;
   __syncthreads();
   const uint32_t C = L.offs[nslices];
   auto at = [&](uint32_t i) -> uint64_t {  // flat candidate i: binary search over the offsets
@@ -238,53 +240,109 @@ __global__ __launch_bounds__(SMP_T) void k_sample(const float *logits, const uin
       }
     }
   };
+  each([&](bool ok, uint64_t c) { if (ok) atomicAdd(&L.hist[c >> 52], 1u); });
+  __syncthreads();
+  // refine until the bin holding the K-th largest, and everything above it, fits in LDS
+  uint64_t prefix = 0;   // composite bits fixed so far
+  uint32_t shift = 52;   // the current field starts here: 12 bits, the last one 4 (bits 3..0)
+  uint32_t above = 0;    // candidates above the current prefix range: all in the top K
+  for (;;) {
+    find_bin<SMP_T, SMP_BINS>(L.hist, above, K, L.wsum, &L.bin, &L.above);
+    const uint32_t bin = L.bin;
+    above = L.above;
+    const uint32_t inbin = L.hist[bin];
+    prefix |= (uint64_t)bin << shift;
+    __syncthreads();
+    if (above + inbin <= SMP_CAND || shift == 0) break;
+    const uint32_t nshift = shift >= 12 ? shift - 12 : 0;
+    const uint64_t hi_mask = ~((1ull << shift) - 1);                   // bits fixed so far
+    const uint32_t fmask = shift >= 12 ? 0xFFFu : (1u << shift) - 1;  // the next field's width
+    for (uint32_t b = tid; b < SMP_BINS; b += SMP_T) L.hist[b] = 0;
+    __syncthreads();
+    each([&](bool ok, uint64_t c) {
+      if (ok && (c & hi_mask) == prefix) atomicAdd(&L.hist[(uint32_t)((c >> nshift) & fmask)], 1u);
+    });
+    __syncthreads();
+    shift = nshift;
+  }
+  // every candidate at or above the selected bin's range start (prefix: zeros below it)
+  if (tid == 0) L.ncand = 0;
+  __syncthreads();
+  each([&](bool ok, uint64_t c) { put(ok && c >= prefix, c); });
+  __syncthreads();
+}
+
+// The token from the slices' candidates; st (optional) receives it as k_argmax_advance would.
+__global__ __launch_bounds__(SMP_T) void k_sample(const float *logits, const uint64_t *cand, const SliceOut *so,
+                                                  uint32_t nslices, uint32_t slice, const SampleParams *prm,
+                                                  int32_t index, StepState *st, int32_t *out, int32_t *tokens,
+                                                  uint32_t cap, int advance) {
+  __shared__ SampleLds L;
+  const uint32_t tid = threadIdx.x, lane = tid & 63;
+  const SampleParams p = *prm;
+  // the slices' totals and best composites, and this wavefront's slices' first 64 candidates
+  // (slices wv, wv + 16, ...; a list has room for more than 64, entries past its count are not used)
+  const uint32_t wv = tid >> 6;
+  const SliceOut mine_so = tid < nslices ? so[tid] : SliceOut{0, 0, 0};
+  constexpr uint32_t WV = SMP_T / 64, SR = SL_MAX / WV;
+  uint64_t first[SR];
+#pragma unroll
+  for (uint32_t r = 0; r < SR; r++) {
+    const uint32_t w = r * WV + wv;
+    first[r] = w < nslices ? cand[(uint64_t)w * slice + lane] : 0;
+  }
+  if (tid < SL_MAX) { L.top[tid] = mine_so.best; L.counts[tid] = mine_so.count; }
+  uint32_t cnt = wave_sum_u32(mine_so.finite);
+  uint64_t best = wave_max_u64(mine_so.best);
+  if (lane == 0) { L.wsum[wv] = cnt; L.wmax[wv] = best; }
+  if (tid == 0) { L.ncand = 0; L.bound = 0; L.cutoff = 0xFFFFFFFFu; }
+  __syncthreads();
+  cnt = 0; best = 0;
+  for (uint32_t u = 0; u < SMP_T / 64; u++) {
+    cnt += L.wsum[u];
+    best = L.wmax[u] > best ? L.wmax[u] : best;
+  }
+  // the candidates that this wavefront takes, into L.cand (uniform control flow)
+  auto put = [&](bool take, uint64_t c) {
+    const uint64_t m = __ballot(take);
+    if (m) {
+      uint32_t slot0 = 0;
+      if (lane == 0) slot0 = atomicAdd(&L.ncand, (uint32_t)__popcll(m));
+      slot0 = __shfl(slot0, 0);
+      const uint32_t slot = slot0 + (uint32_t)__popcll(m & ((1ull << lane) - 1));
+      if (take && slot < SMP_CAND) L.cand[slot] = c;
+    }
+  };
   int32_t token = -1;
   if (cnt > 0 && p.temperature == 0.0) {
     token = (int32_t)comp_index(best);
   } else if (cnt > 0) {
     const uint32_t K = p.top_k < cnt ? p.top_k : cnt;
-    for (uint32_t b = tid; b < SMP_BINS; b += SMP_T) L.hist[b] = 0;
-    __syncthreads();
-    each([&](bool ok, uint64_t c) { if (ok) atomicAdd(&L.hist[c >> 52], 1u); });
-    __syncthreads();
-    // refine until the bin holding the K-th largest, and everything above it, fits in LDS
-    uint64_t prefix = 0;   // composite bits fixed so far
-    uint32_t shift = 52;   // the current field starts here: 12 bits, the last one 4 (bits 3..0)
-    uint32_t above = 0;    // candidates above the current prefix range: all in the top K
-    for (;;) {
-      find_bin<SMP_T, SMP_BINS>(L.hist, above, K, L.wsum, &L.bin, &L.above);
-      const uint32_t bin = L.bin;
-      above = L.above;
-      const uint32_t inbin = L.hist[bin];
-      prefix |= (uint64_t)bin << shift;
-      __syncthreads();
-      if (above + inbin <= SMP_CAND || shift == 0) break;
-      const uint32_t nshift = shift >= 12 ? shift - 12 : 0;
-      const uint64_t hi_mask = ~((1ull << shift) - 1);                   // bits fixed so far
-      const uint32_t fmask = shift >= 12 ? 0xFFFu : (1u << shift) - 1;  // the next field's width
-      for (uint32_t b = tid; b < SMP_BINS; b += SMP_T) L.hist[b] = 0;
-      __syncthreads();
-      each([&](bool ok, uint64_t c) {
-        if (ok && (c & hi_mask) == prefix) atomicAdd(&L.hist[(uint32_t)((c >> nshift) & fmask)], 1u);
-      });
-      __syncthreads();
-      shift = nshift;
-    }
-    // every candidate at or above the selected bin's range start (prefix: zeros below it)
-    if (tid == 0) L.ncand = 0;
-    __syncthreads();
-    each([&](bool ok, uint64_t c) {
-      const bool take = ok && c >= prefix;
-      const uint64_t m = __ballot(take);
-      if (m) {
-        uint32_t slot0 = 0;
-        if (lane == 0) slot0 = atomicAdd(&L.ncand, (uint32_t)__popcll(m));
-        slot0 = __shfl(slot0, 0);
-        const uint32_t slot = slot0 + (uint32_t)__popcll(m & ((1ull << lane) - 1));
-        if (take && slot < SMP_CAND) L.cand[slot] = c;
+    bool gathered = false;
+    if (K <= nslices) {
+      // the K-th largest best: the one with K - 1 larger (zeros, slices without a finite
+      // logit, are below every composite; with fewer than K bests the bound stays 0)
+      if (tid < nslices && mine_so.best) {
+        uint32_t larger = 0;
+#pragma unroll 8
+        for (uint32_t j = 0; j < nslices; j++) larger += L.top[j] > mine_so.best ? 1u : 0u;
+        if (larger == K - 1) L.bound = mine_so.best;
       }
-    });
-    __syncthreads();
+      __syncthreads();
+      const uint64_t bound = L.bound;
+#pragma unroll
+      for (uint32_t r = 0; r < SR; r++) {
+        const uint32_t w = r * WV + wv, n = w < nslices ? L.counts[w] : 0;
+        put(lane < n && first[r] >= bound, first[r]);
+        for (uint32_t i0 = 64; i0 < n; i0 += 64) {
+          const uint64_t c = i0 + lane < n ? cand[(uint64_t)w * slice + i0 + lane] : 0;
+          put(i0 + lane < n && c >= bound, c);
+        }
+      }
+      __syncthreads();
+      gathered = L.ncand <= SMP_CAND;
+    }
+    if (!gathered) select(L, cand, slice, nslices, K, put);
     // rank sort, descending: the composites are unique, so each one's place is the count of
     // larger ones
     const uint32_t nc = L.ncand < SMP_CAND ? L.ncand : SMP_CAND;
@@ -298,26 +356,44 @@ __global__ __launch_bounds__(SMP_T) void k_sample(const float *logits, const uin
     if (tid < nc) L.cand[rank] = mine;
     __syncthreads();
     // probabilities of the top K (f64, as the reference's numbers)
-    const double bestv = (double)logits[comp_index(best)];
-    if (tid < K) L.prob[tid] = exp(((double)logits[comp_index(L.cand[tid])] - bestv) / p.temperature);
+    if (tid < K) L.prob[tid] = exp(((double)comp_value(L.cand[tid]) - (double)comp_value(best)) / p.temperature);
     __syncthreads();
     if (tid == 0) {
-      double total = 0.0;
-      for (uint32_t j = 0; j < K; j++) total += L.prob[j];
-      double retained = 0.0;
-      uint32_t cutoff = 0;
-      for (; cutoff < K; cutoff++) {
-        retained += L.prob[cutoff];
-        if (retained / total >= p.top_p) { cutoff++; break; }
+      double sum = 0.0;
+      for (uint32_t j0 = 0; j0 < K; j0 += 8) {  // K <= 200, prob and cum hold 256
+        double q[8];
+#pragma unroll
+        for (uint32_t e = 0; e < 8; e++) q[e] = L.prob[j0 + e];
+#pragma unroll
+        for (uint32_t e = 0; e < 8; e++) {
+          sum += q[e];
+          L.cum[j0 + e] = sum;
+        }
       }
+    }
+    __syncthreads();
+    // the shortest prefix whose share reaches top-p (all K where none does): a share never
+    // falls along the prefix, so the first is the least index of those that reach it
+    if (tid < K && L.cum[tid] / L.cum[K - 1] >= p.top_p) atomicMin(&L.cutoff, tid + 1);
+    __syncthreads();
+    if (tid == 0) {
+      const uint32_t cutoff = L.cutoff < K ? L.cutoff : K;
       const int64_t at_pos = index >= 0 ? (int64_t)index : (int64_t)st->pos + 1;
       const double u = (double)(splitmix64_at(p.seed, (uint64_t)at_pos) >> 11) * 0x1.0p-53;
-      double draw = u * retained;
+      double draw = u * L.cum[cutoff - 1];
       token = (int32_t)comp_index(best);
-      for (uint32_t j = 0; j < cutoff; j++) {
-        draw -= L.prob[j];
-        if (draw <= 0.0) { token = (int32_t)comp_index(L.cand[j]); break; }
+      uint32_t at = cutoff;  // no early exit: the loads of a chunk go out together
+      for (uint32_t j0 = 0; j0 < cutoff && at == cutoff; j0 += 8) {
+        double q[8];
+#pragma unroll
+        for (uint32_t e = 0; e < 8; e++) q[e] = L.prob[j0 + e];  // within prob; entries past the cutoff are not used
+#pragma unroll
+        for (uint32_t e = 0; e < 8; e++) {
+          draw -= q[e];
+          if (draw <= 0.0 && at == cutoff && j0 + e < cutoff) at = j0 + e;
+        }
       }
+      if (at < cutoff) token = (int32_t)comp_index(L.cand[at]);
     }
   }
   if (tid != 0) return;
