@@ -28,7 +28,7 @@ struct wgd_context {
   uint64_t gemm_part_floats = 0;
   uint8_t *gemm_xs = nullptr;        // its input split into f16 (hi, lo)
   uint64_t gemm_xs_bytes = 0;
-  wgd::SampleParams *sample_params = nullptr;  // settings of wgd_sample
+  int32_t *sample_result = nullptr;            // the token of wgd_sample, in pinned host memory
   void *sample_scratch = nullptr;              // its slices' candidates
   uint64_t sample_scratch_bytes = 0;
 };

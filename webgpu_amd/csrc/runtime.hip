@@ -141,6 +141,7 @@ void wgd_destroy(wgd_context *ctx) {
   ctx->buffers.clear();
   for (auto &kv : ctx->sizes) hipFree(kv.first);
   ctx->sizes.clear();
+  if (ctx->sample_result) hipHostFree(ctx->sample_result);
   hipStreamDestroy(ctx->stream);
   delete ctx;
 }
@@ -615,12 +616,12 @@ int wgd_sample(wgd_context *ctx, const wgd_buffer *logits, uint32_t n, double te
   if (!token || !n || index > 0x7FFFFFFFu) return fail(ctx, WGD_E_INVALID, "wgd_sample: bad arguments");
   if (!(temperature >= 0.0 && temperature <= 2.0) || top_k < 1 || top_k > 200 || !(top_p > 0.0 && top_p <= 1.0))
     return fail(ctx, WGD_E_INVALID, "Invalid sampling settings.");
-  if (!ctx->sample_params) {
-    int rc = ctx_alloc(ctx, sizeof(SampleParams), "sampling settings", (void **)&ctx->sample_params);
-    if (rc) return rc;
-  }
+  // The settings travel with the launches and the kernel stores the token into pinned host
+  // memory, so a draw is two launches and one wait, without a copy either way.
+  int rc = WGD_OK;
+  if (!ctx->sample_result)
+    rc = ctx_check(ctx, hipHostMalloc((void **)&ctx->sample_result, sizeof(int32_t), hipHostMallocDefault), "sample");
   const SampleParams p = {temperature, top_p, top_k, 0, seed};
-  int rc = ctx_check(ctx, hipMemcpyAsync(ctx->sample_params, &p, sizeof p, hipMemcpyHostToDevice, ctx->stream), "sample");
   if (!rc && ctx->sample_scratch_bytes < sample_scratch_bytes(n)) {
     if (ctx->sample_scratch) ctx_free(ctx, ctx->sample_scratch);
     ctx->sample_scratch = nullptr;
@@ -628,13 +629,11 @@ int wgd_sample(wgd_context *ctx, const wgd_buffer *logits, uint32_t n, double te
     rc = ctx_alloc(ctx, sample_scratch_bytes(n), "sampling candidates", &ctx->sample_scratch);
     if (!rc) ctx->sample_scratch_bytes = sample_scratch_bytes(n);
   }
-  if (!rc) rc = ctx_check(ctx, sample(ctx->stream, (const float *)logits->ptr, n, ctx->sample_params, (int32_t)index,
-                                      nullptr, ctx->argmax_scratch, nullptr, 0, false, ctx->sample_scratch), "sample");
+  if (!rc) rc = ctx_check(ctx, sample(ctx->stream, (const float *)logits->ptr, n, nullptr, (int32_t)index, nullptr,
+                                      ctx->sample_result, nullptr, 0, false, ctx->sample_scratch, &p), "sample");
   if (!rc) rc = ctx_sync(ctx, "sample");
   if (rc) return rc;
-  int32_t id = -1;
-  hipError_t e = hipMemcpy(&id, ctx->argmax_scratch, 4, hipMemcpyDeviceToHost);
-  if (e != hipSuccess) return hip_fail(ctx, e, "sample read-back");
+  const int32_t id = *(volatile int32_t *)ctx->sample_result;
   *token = id;
   if (id < 0) return fail(ctx, WGD_E_NONFINITE, "Inference produced non-finite logits. Stop and report this model/runtime combination.");
   return WGD_OK;

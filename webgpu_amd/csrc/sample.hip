@@ -113,7 +113,8 @@ __device__ __forceinline__ void find_bin(const uint32_t *hist, uint32_t above, u
 struct SliceOut { uint64_t best; uint32_t finite, count; };
 
 __global__ __launch_bounds__(SL_T) void k_sample_local(const float *logits, uint32_t n, uint32_t slice,
-                                                       const SampleParams *prm, uint64_t *cand, SliceOut *so) {
+                                                       const SampleParams *prm, SampleParams value, uint64_t *cand,
+                                                       SliceOut *so) {
   __shared__ uint32_t hist[SMP_BINS];
   __shared__ uint32_t wsum[SL_T / 64];
   __shared__ uint64_t wmax[SL_T / 64];
@@ -153,7 +154,7 @@ __global__ __launch_bounds__(SL_T) void k_sample_local(const float *logits, uint
     cnt += wsum[u];
     best = wmax[u] > best ? wmax[u] : best;
   }
-  const SampleParams p = *prm;
+  const SampleParams p = prm ? *prm : value;
   const uint32_t K = p.top_k < cnt ? p.top_k : cnt;
   const bool gather = p.temperature != 0.0 && K > 0;
   if (gather) {
@@ -275,11 +276,11 @@ __device__ __forceinline__ void select(SampleLds &L, const uint64_t *cand, uint3
 // The token from the slices' candidates; st (optional) receives it as k_argmax_advance would.
 __global__ __launch_bounds__(SMP_T) void k_sample(const float *logits, const uint64_t *cand, const SliceOut *so,
                                                   uint32_t nslices, uint32_t slice, const SampleParams *prm,
-                                                  int32_t index, StepState *st, int32_t *out, int32_t *tokens,
+                                                  SampleParams value, int32_t index, StepState *st, int32_t *out, int32_t *tokens,
                                                   uint32_t cap, int advance) {
   __shared__ SampleLds L;
   const uint32_t tid = threadIdx.x, lane = tid & 63;
-  const SampleParams p = *prm;
+  const SampleParams p = prm ? *prm : value;
   // the slices' totals and best composites, and this wavefront's slices' first 64 candidates
   // (slices wv, wv + 16, ...; a list has room for more than 64, entries past its count are not used)
   const uint32_t wv = tid >> 6;
@@ -425,16 +426,18 @@ uint64_t sample_scratch_bytes(uint32_t n) {
 }
 
 hipError_t sample(hipStream_t s, const float *logits, uint32_t n, const SampleParams *params, int32_t index,
-                  StepState *st, int32_t *out, int32_t *tokens, uint32_t cap, bool advance, void *scratch) {
-  if (!n || !scratch || (index < 0 && !st) || (advance && (!st || !tokens))) return hipErrorInvalidValue;
+                  StepState *st, int32_t *out, int32_t *tokens, uint32_t cap, bool advance, void *scratch,
+                  const SampleParams *host_params) {
+  if (!n || !scratch || (!params && !host_params) || (index < 0 && !st) || (advance && (!st || !tokens))) return hipErrorInvalidValue;
+  const SampleParams value = host_params ? *host_params : SampleParams{};
   uint32_t ns, sl;
   slicing(n, &ns, &sl);
   uint64_t *cand = (uint64_t *)scratch;
   SliceOut *so = (SliceOut *)((uint8_t *)scratch + cand_bytes(ns, sl));
-  hipLaunchKernelGGL(k_sample_local, dim3(ns), dim3(SL_T), 0, s, logits, n, sl, params, cand, so);
+  hipLaunchKernelGGL(k_sample_local, dim3(ns), dim3(SL_T), 0, s, logits, n, sl, params, value, cand, so);
   WGD_HIP(hipGetLastError());
   hipLaunchKernelGGL(k_sample, dim3(1), dim3(SMP_T), 0, s, logits, (const uint64_t *)cand, (const SliceOut *)so, ns,
-                     sl, params, index, st, out, tokens, cap, advance ? 1 : 0);
+                     sl, params, value, index, st, out, tokens, cap, advance ? 1 : 0);
   return hipGetLastError();
 }
 
