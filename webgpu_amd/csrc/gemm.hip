@@ -313,12 +313,12 @@ __device__ __forceinline__ f16x2 fma2(f16x2 a, f16x2 b, f16x2 c) { return __buil
 __device__ __forceinline__ f16x8 oct(f16x2 a, f16x2 b, f16x2 c, f16x2 d) {
   return __builtin_bit_cast(f16x8, make_uint4(u32(a), u32(b), u32(c), u32(d)));
 }
-// The 6-bit scale and min of the sub-block of chunk lane group g in unit parity odd (quant.ts:9-12).
+// The 6-bit scale and min of chunk g of a unit, the first (odd = 0) or second of its block
+// (quant.ts:9-12).
 __device__ __forceinline__ void scale_min(const uint4 &h, uint32_t odd, uint32_t g, uint32_t &sc, uint32_t &m) {
   const uint32_t sh = 8 * g, A = h.y >> sh, B = h.z >> sh, C = h.w >> sh;
-  const uint32_t o = 0u - odd;  // selects, not branches: odd is uniform and known only at run time
-  sc = (((C & 15u) | ((A >> 2) & 48u)) & o) | (A & 63u & ~o);
-  m = ((((C >> 4) & 15u) | ((B >> 2) & 48u)) & o) | (B & 63u & ~o);
+  sc = odd ? (C & 15u) | ((A >> 2) & 48u) : A & 63u;
+  m = odd ? ((C >> 4) & 15u) | ((B >> 2) & 48u) : B & 63u;
 }
 
 // A lane's weights of 16 rows x one 128-column unit. fetch() loads them; unpack() leaves the MFMA
@@ -333,9 +333,9 @@ template <> struct QUnit<Q4_K> {
     q = qld16(rw, ((T * a.C + 4 * u + g) * 16 + c) * 16);
     h = qld16(rw, a.nbp * 128 + ((T * a.bpr + u / 2) * 16 + c) * 16);
   }
-  __device__ void unpack(uint32_t u, uint32_t g, f16x8 *w, f16x8 *, float *d, float &mn) const {
+  __device__ void unpack(uint32_t odd, uint32_t g, f16x8 *w, f16x8 *, float *d, float &mn) const {
     uint32_t sc, m;
-    scale_min(h, u & 1, g, sc, m);
+    scale_min(h, odd, g, sc, m);
     d[0] = f16_lo(h.x);
     mn = -f16_lo(h.x >> 16) * (float)m;
     // low nibbles as 1024 + q, high nibbles (bits 4-7 of the mantissa, in units of 1/16 at 64) as 64 + q:
@@ -361,9 +361,9 @@ template <> struct QUnit<Q5_K> {
     b = __builtin_amdgcn_raw_buffer_load_b32(rw, a.nbp * 128 + tc * 4, 0, 0);
     h = qld16(rw, a.nbp * 160 + ((T * a.bpr + u / 2) * 16 + c) * 16);
   }
-  __device__ void unpack(uint32_t u, uint32_t g, f16x8 *w, f16x8 *, float *d, float &mn) const {
+  __device__ void unpack(uint32_t odd, uint32_t g, f16x8 *w, f16x8 *, float *d, float &mn) const {
     uint32_t sc, m;
-    scale_min(h, u & 1, g, sc, m);
+    scale_min(h, odd, g, sc, m);
     d[0] = f16_lo(h.x);
     mn = -f16_lo(h.x >> 16) * (float)m;
     const f16x2 s = both((_Float16)(uint16_t)sc), bl = s * both((_Float16)-1024.f);
@@ -472,9 +472,11 @@ template <> struct QUnit<Q4_0> {
 // the LDS reads of the activations per MFMA.
 constexpr uint32_t qg_rt(uint32_t tt) { return tt <= 2 ? 1 : 2; }
 constexpr uint32_t qg_threads(uint32_t tt) { return QG_M / 16 / qg_rt(tt) * 64; }
-// Units of weights in flight per row tile (registers), and units of activations per LDS buffer (17 to 34 KB).
-constexpr uint32_t qg_depth(int type, uint32_t tt) { return type == Q8_0 || type == Q4_0 ? (tt <= 2 ? 2 : 1) : tt <= 2 ? 4 : 2; }
-constexpr uint32_t qg_stage(int type, uint32_t tt) { return 4 / tt < qg_depth(type, tt) ? 4 / tt : qg_depth(type, tt); }
+// Units of weights in flight per row tile (registers), and units of activations per LDS buffer (17 to
+// 34 KB). Two units suffice with eight wavefronts or more a CU; four and eight were slower
+// (28672 x 4096 Q4_K, 16 tokens: 20.5, 21.5 and 28.8 us), their registers and prologue cost more.
+constexpr uint32_t qg_depth(int type, uint32_t tt) { return tt == 4 && (type == Q8_0 || type == Q4_0) ? 1 : 2; }
+constexpr uint32_t qg_stage(int type, uint32_t tt) { return tt == 4 ? 1 : qg_depth(type, tt); }
 
 template <int TYPE, uint32_t TT>
 __device__ __forceinline__ void gemm_tile(const QGemm &a, const QJob &jb, uint32_t mt, uint8_t *lds) {
@@ -525,7 +527,7 @@ __device__ __forceinline__ void gemm_tile(const QGemm &a, const QJob &jb, uint32
     f16x8 w[RT][4], wl[RT][W::LO ? 4 : 1];
     float dr[RT][W::CHUNK ? 1 : 4], mn[RT];
 #pragma unroll
-    for (uint32_t r = 0; r < RT; r++) buf[d][r].unpack(u, g, w[r], wl[r], dr[r], mn[r]);
+    for (uint32_t r = 0; r < RT; r++) buf[d][r].unpack(d % 2, g, w[r], wl[r], dr[r], mn[r]);
 #pragma unroll
     for (uint32_t t = 0; t < TT; t++) {
       const uint8_t *xb = xl + t * SPLIT_BLOCK;
@@ -745,12 +747,12 @@ bool gemm_group_ok(const GemmGroup &g, uint32_t batch) {
 static uint32_t token_blocks(uint32_t batch) { return batch <= 16 ? 1 : batch <= 32 ? 2 : 4; }
 static uint32_t token_tiles(uint32_t batch) { return (batch + 16 * token_blocks(batch) - 1) / (16 * token_blocks(batch)); }
 
-// K span per workgroup: enough splits for two workgroups per CU, each at least one unit, and
+// K span per workgroup: splits until the launch fills its workgroup slots, each at least two units, and
 // no more partial sums than the scratch holds.
 static uint32_t group_kspan(const GemmGroup &g, uint32_t batch, uint64_t scratch_floats, uint32_t *rows_total) {
-  // splits end on units (each chunk reads its own block's header, so a split may start
-  // inside a 256-column super-block): finer splits fill the chip closer to its target
-  const uint32_t align = QG_U;
+  // splits end on pairs of units, a K-quant's block, so the kernel knows at compile time which half
+  // of a block a unit is
+  const uint32_t align = 2 * QG_U;
   uint32_t tiles = 0, rows = 0;
   for (uint32_t j = 0; j < g.n; j++) {
     const Matrix &w = *g.job[j].w;
@@ -759,9 +761,15 @@ static uint32_t group_kspan(const GemmGroup &g, uint32_t batch, uint64_t scratch
   }
   tiles *= token_tiles(batch);
   *rows_total = rows;
-  const uint32_t cols = g.job[0].w->cols, target = 2 * (uint32_t)device_cu_count();
+  // Up to 32 tokens, where the rows give at most half a workgroup per CU, the splits stop at one
+  // workgroup (eight wavefronts) per CU: fewer partial sums, the same or less time (16 tokens: 4096 x
+  // 4096 7.9 -> 7.0 us, 6144 x 4096 10.1 -> 8.8, 4096 x 14336 13.9 -> 13.6). Taller matrices would be left
+  // with one long split (28672 x 4096: 22.2 us against 20.5 in two), 64 tokens with less to
+  // overlap (4096 x 14336 31.8 against 28.8).
+  const uint32_t cus = (uint32_t)device_cu_count(), cols = g.job[0].w->cols;
+  const uint32_t target = token_blocks(batch) <= 2 && 2 * tiles <= cus ? cus : 2 * cus;
   uint32_t splits = tiles >= target ? 1 : target / tiles;
-  const uint32_t units = split_kblocks(cols);
+  const uint32_t units = (cols + align - 1) / align;
   if (splits > units) splits = units;
   if (splits > 16) splits = 16;
   // The workgroups run in rounds of `target` slots, and a short last round leaves CUs idle
