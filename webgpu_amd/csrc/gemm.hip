@@ -260,7 +260,7 @@ constexpr uint32_t QG_U = SPLIT_K;   // columns of a unit
 struct QJob {
   const uint8_t *w; uint32_t wbytes;
   uint32_t C, bpr, nbp;  // chunk columns, blocks per row, blocks of the padded matrix
-  uint32_t rows, tiles, kind, row0;
+  uint32_t rows, tiles, kind, row0, off;  // off: the launch's tiles before this matrix's, mod 8
   float *y; uint32_t stride, row_base;
 };
 constexpr uint32_t QG_MAX_JOBS = 3;
@@ -471,19 +471,29 @@ template <> struct QUnit<Q4_0> {
 // than four of two (8B prompt in 16s 6.22 against 6.34 ms); for 64 tokens two row tiles halve
 // the LDS reads of the activations per MFMA.
 constexpr uint32_t qg_rt(uint32_t tt) { return tt <= 2 ? 1 : 2; }
-constexpr uint32_t qg_threads(uint32_t tt) { return QG_M / 16 / qg_rt(tt) * 64; }
+// Rows per workgroup: 128, and 256 (eight wavefronts) where it takes 128 tokens.
+constexpr uint32_t qg_rows(uint32_t tt) { return tt == 8 ? 2 * QG_M : QG_M; }
+constexpr uint32_t qg_threads(uint32_t tt) { return qg_rows(tt) / 16 / qg_rt(tt) * 64; }
 // Units of weights in flight per row tile (registers), and units of activations per LDS buffer (17 to
 // 34 KB). Two units suffice with eight wavefronts or more a CU; four and eight were slower
 // (28672 x 4096 Q4_K, 16 tokens: 20.5, 21.5 and 28.8 us), their registers and prologue cost more.
-constexpr uint32_t qg_depth(int type, uint32_t tt) { return tt == 4 && (type == Q8_0 || type == Q4_0) ? 1 : 2; }
-constexpr uint32_t qg_stage(int type, uint32_t tt) { return tt == 4 ? 1 : qg_depth(type, tt); }
+constexpr uint32_t qg_depth(int type, uint32_t tt) { return tt == 8 || (tt == 4 && (type == Q8_0 || type == Q4_0)) ? 1 : 2; }
+constexpr uint32_t qg_stage(int type, uint32_t tt) { return tt >= 4 ? 1 : qg_depth(type, tt); }
 
 template <int TYPE, uint32_t TT>
 __device__ __forceinline__ void gemm_tile(const QGemm &a, const QJob &jb, uint32_t mt, uint8_t *lds) {
   constexpr uint32_t RT = qg_rt(TT), D = qg_depth(TYPE, TT), S = qg_stage(TYPE, TT), UB = TT * SPLIT_BLOCK, NT = qg_threads(TT);
   typedef QUnit<TYPE> W;
   const uint32_t tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, g = lane >> 4, c = lane & 15;
-  const uint32_t m0 = mt * QG_M + wv * 16 * RT, b0 = blockIdx.y * TT, z = blockIdx.z;
+  uint32_t m0 = mt * QG_M + wv * 16 * RT;
+  if constexpr (qg_rows(TT) == 2 * QG_M) {
+    // Two runs of 128 rows. The finishes expect run r on XCD r % 8 (as 128-row tiles put it), so of every
+    // eight whole tiles, on XCDs off, off + 1, ..., tile t takes the runs r and r + 8 with r = t's XCD.
+    const uint32_t half = wv >> 2, t8 = mt / 8 * 8;
+    const uint32_t run = t8 + 8 <= jb.tiles ? 2 * t8 + (mt + jb.off) % 8 + 8 * half : 2 * mt + half;
+    m0 = run * QG_M + (wv & 3) * 16 * RT;
+  }
+  const uint32_t b0 = blockIdx.y * TT, z = blockIdx.z;
   const uint32_t kbs = split_kblocks(a.cols);
   const uint32_t u0 = z * (a.kspan / QG_U), ue = u0 + a.kspan / QG_U, u1 = ue < kbs ? ue : kbs;
   const uint32_t T0 = m0 / 16;
@@ -527,7 +537,7 @@ __device__ __forceinline__ void gemm_tile(const QGemm &a, const QJob &jb, uint32
     f16x8 w[RT][4], wl[RT][W::LO ? 4 : 1];
     float dr[RT][W::CHUNK ? 1 : 4], mn[RT];
 #pragma unroll
-    for (uint32_t r = 0; r < RT; r++) buf[d][r].unpack(d % 2, g, w[r], wl[r], dr[r], mn[r]);
+    for (uint32_t r = 0; r < RT; r++) buf[d][r].unpack(D > 1 ? d % 2 : u % 2, g, w[r], wl[r], dr[r], mn[r]);
 #pragma unroll
     for (uint32_t t = 0; t < TT; t++) {
       const uint8_t *xb = xl + t * SPLIT_BLOCK;
@@ -741,25 +751,37 @@ bool gemm_group_ok(const GemmGroup &g, uint32_t batch) {
   return group_types(g, t) && qgemm_pair(t[0], t[1]);
 }
 
-// 16-token blocks of a workgroup: the smallest of 1, 2, 4 that covers the batch. 65 to 128
-// tokens take two workgroups of 64: with 128 in one, its accumulators leave no registers to load
-// the next activations early (8B prefill in batches of 128: 4.32 against 3.74 ms).
-static uint32_t token_blocks(uint32_t batch) { return batch <= 16 ? 1 : batch <= 32 ? 2 : 4; }
-static uint32_t token_tiles(uint32_t batch) { return (batch + 16 * token_blocks(batch) - 1) / (16 * token_blocks(batch)); }
+// 16-token blocks of a workgroup: the smallest of 1, 2, 4 that covers the batch; past 64 tokens
+// workgroups of 64 each. K-quant groups of one type whose 128-row tiles fill half the CUs or
+// more take 8: workgroups of 256 rows x 128 tokens, which unpack each weight once (28672 x 4096,
+// 128 tokens: Q4_K 93.7 -> 88.2 us, Q6_K 131.5 -> 111.8). Shorter matrices need the smaller
+// workgroups (4096 x 4096: 18.4 against 22.3), and the 32-column types the registers (Q8_0
+// 100 against 122.5).
+static uint32_t token_blocks(const GemmGroup &g, uint32_t batch) {
+  if (batch <= 16) return 1;
+  if (batch <= 64) return batch <= 32 ? 2 : 4;
+  uint32_t tiles = 0;
+  for (uint32_t j = 0; j < g.n; j++) {
+    const int t = g.job[j].w->type;
+    if (t != g.job[0].w->type || t == Q8_0 || t == Q4_0) return 4;
+    tiles += (g.job[j].w->rows + QG_M - 1) / QG_M;
+  }
+  return 2 * tiles >= (uint32_t)device_cu_count() ? 8 : 4;
+}
 
 // K span per workgroup: splits until the launch fills its workgroup slots, each at least two units, and
 // no more partial sums than the scratch holds.
 static uint32_t group_kspan(const GemmGroup &g, uint32_t batch, uint64_t scratch_floats, uint32_t *rows_total) {
   // splits end on pairs of units, a K-quant's block, so the kernel knows at compile time which half
   // of a block a unit is
-  const uint32_t align = 2 * QG_U;
+  const uint32_t align = 2 * QG_U, tb = token_blocks(g, batch);
   uint32_t tiles = 0, rows = 0;
   for (uint32_t j = 0; j < g.n; j++) {
     const Matrix &w = *g.job[j].w;
-    tiles += (w.rows + QG_M - 1) / QG_M;
+    tiles += (w.rows + qg_rows(tb) - 1) / qg_rows(tb);
     rows += w.rows;
   }
-  tiles *= token_tiles(batch);
+  tiles *= (batch + 16 * tb - 1) / (16 * tb);
   *rows_total = rows;
   // Up to 32 tokens, where the rows give at most half a workgroup per CU, the splits stop at one
   // workgroup (eight wavefronts) per CU: fewer partial sums, the same or less time (16 tokens: 4096 x
@@ -767,7 +789,7 @@ static uint32_t group_kspan(const GemmGroup &g, uint32_t batch, uint64_t scratch
   // with one long split (28672 x 4096: 22.2 us against 20.5 in two), 64 tokens with less to
   // overlap (4096 x 14336 31.8 against 28.8).
   const uint32_t cus = (uint32_t)device_cu_count(), cols = g.job[0].w->cols;
-  const uint32_t target = token_blocks(batch) <= 2 && 2 * tiles <= cus ? cus : 2 * cus;
+  const uint32_t target = tb == 8 || (tb <= 2 && 2 * tiles <= cus) ? cus : 2 * cus;  // 8: one fits a CU
   uint32_t splits = tiles >= target ? 1 : target / tiles;
   const uint32_t units = (cols + align - 1) / align;
   if (splits > units) splits = units;
@@ -824,8 +846,10 @@ static void launch_qgemm_tt(hipStream_t s, dim3 grid, const QGemm &q) {
   hipLaunchKernelGGL((k_gemm_q<T0, T1, TT>), grid, dim3(qg_threads(TT)), 2 * S * TT * SPLIT_BLOCK, s, q);
 }
 template <int T0, int T1>
-static void launch_qgemm(hipStream_t s, dim3 grid, const QGemm &q) {
-  switch (token_blocks(q.batch)) {
+static void launch_qgemm(hipStream_t s, dim3 grid, uint32_t tb, const QGemm &q) {
+  if constexpr (T0 == T1 && T0 != Q8_0 && T0 != Q4_0)
+    if (tb == 8) return launch_qgemm_tt<T0, T1, 8>(s, grid, q);
+  switch (tb) {
     case 1: return launch_qgemm_tt<T0, T1, 1>(s, grid, q);
     case 2: return launch_qgemm_tt<T0, T1, 2>(s, grid, q);
     default: return launch_qgemm_tt<T0, T1, 4>(s, grid, q);
@@ -848,6 +872,7 @@ hipError_t gemm_group(hipStream_t s, const GemmGroup &g, const float *x, uint32_
   }
   int types[2];
   group_types(g, types);
+  const uint32_t tb = token_blocks(g, batch);
   QGemm q{};
   q.njobs = g.n; q.xs = scratch->xs; q.cols = cols; q.batch = batch; q.accumulate = g.accumulate ? 1u : 0u;
   uint32_t tiles = 0, row0 = 0;
@@ -858,7 +883,7 @@ hipError_t gemm_group(hipStream_t s, const GemmGroup &g, const float *x, uint32_
     QJob &jb = q.job[j];
     jb.w = w.data; jb.wbytes = (uint32_t)wbytes;
     jb.C = w.cols / chunk_elems(w.type); jb.bpr = w.cols / block_size(w.type); jb.nbp = jb.bpr * (uint32_t)tile_rows(w.rows);
-    jb.rows = w.rows; jb.tiles = (w.rows + QG_M - 1) / QG_M; jb.kind = w.type == types[0] ? 0u : 1u; jb.row0 = row0;
+    jb.rows = w.rows; jb.tiles = (w.rows + qg_rows(tb) - 1) / qg_rows(tb); jb.off = tiles % 8; jb.kind = w.type == types[0] ? 0u : 1u; jb.row0 = row0;
     jb.y = g.job[j].y; jb.stride = g.job[j].stride; jb.row_base = g.job[j].row_base;
     tiles += jb.tiles; row0 += w.rows;
   }
@@ -871,18 +896,18 @@ hipError_t gemm_group(hipStream_t s, const GemmGroup &g, const float *x, uint32_
   if (partials && (splits > MAX_SPLITS || (uint64_t)splits * batch * q.rows_total * 4 >= (1ull << 31)))
     return hipErrorInvalidValue;
   q.part = partials ? scratch->p : nullptr;
-  const dim3 grid(tiles, token_tiles(batch), splits);
+  const dim3 grid(tiles, (batch + 16 * tb - 1) / (16 * tb), splits);
   const int a = types[0], b = types[1];
-  if (a == Q4_K && b == Q4_K) launch_qgemm<Q4_K, Q4_K>(s, grid, q);
-  else if (a == Q6_K && b == Q6_K) launch_qgemm<Q6_K, Q6_K>(s, grid, q);
-  else if (a == Q8_0 && b == Q8_0) launch_qgemm<Q8_0, Q8_0>(s, grid, q);
-  else if (a == Q4_K && b == Q6_K) launch_qgemm<Q4_K, Q6_K>(s, grid, q);
-  else if (a == Q8_0 && b == Q4_K) launch_qgemm<Q8_0, Q4_K>(s, grid, q);
-  else if (a == Q8_0 && b == Q6_K) launch_qgemm<Q8_0, Q6_K>(s, grid, q);
-  else if (a == Q5_K && b == Q5_K) launch_qgemm<Q5_K, Q5_K>(s, grid, q);
-  else if (a == Q4_0 && b == Q4_0) launch_qgemm<Q4_0, Q4_0>(s, grid, q);
-  else if (a == Q4_K && b == Q5_K) launch_qgemm<Q4_K, Q5_K>(s, grid, q);
-  else if (a == Q5_K && b == Q6_K) launch_qgemm<Q5_K, Q6_K>(s, grid, q);
+  if (a == Q4_K && b == Q4_K) launch_qgemm<Q4_K, Q4_K>(s, grid, tb, q);
+  else if (a == Q6_K && b == Q6_K) launch_qgemm<Q6_K, Q6_K>(s, grid, tb, q);
+  else if (a == Q8_0 && b == Q8_0) launch_qgemm<Q8_0, Q8_0>(s, grid, tb, q);
+  else if (a == Q4_K && b == Q6_K) launch_qgemm<Q4_K, Q6_K>(s, grid, tb, q);
+  else if (a == Q8_0 && b == Q4_K) launch_qgemm<Q8_0, Q4_K>(s, grid, tb, q);
+  else if (a == Q8_0 && b == Q6_K) launch_qgemm<Q8_0, Q6_K>(s, grid, tb, q);
+  else if (a == Q5_K && b == Q5_K) launch_qgemm<Q5_K, Q5_K>(s, grid, tb, q);
+  else if (a == Q4_0 && b == Q4_0) launch_qgemm<Q4_0, Q4_0>(s, grid, tb, q);
+  else if (a == Q4_K && b == Q5_K) launch_qgemm<Q4_K, Q5_K>(s, grid, tb, q);
+  else if (a == Q5_K && b == Q6_K) launch_qgemm<Q5_K, Q6_K>(s, grid, tb, q);
   else return hipErrorInvalidValue;
   WGD_HIP(hipGetLastError());
   if (g.glu_out) {
