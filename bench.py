@@ -18,8 +18,8 @@ same microbench (profiles/k_mv_matvec_microbench.md). The other microbench shape
 prefill_tok_s: the 512-token prompt after one untimed pass, median of three passes.
 prefill_gemm: the prompt-batch dequant-GEMM at the 8B layer shapes with 128 tokens as
 single-matrix wgd_matmul calls (input split, GEMM and split-K reduction), timed with HIP
-events; its MFMA utilisation counts the three bf16 MFMAs per product of the hi/lo operand
-split against the 2.5 PFLOP/s dense bf16 peak.
+events; its MFMA utilisation counts the f16 MFMAs per product (hi and lo activations: two, three for Q6_K's
+weight pairs) against the 2.5 PFLOP/s dense 16-bit peak.
 
 cpu_baseline: the float64 C oracle (OpenMP over the host cores) decoding the same 8B
 model on a bounded sample (8-token prompt, then as many greedy tokens as fit ~15 s).
@@ -211,15 +211,15 @@ def probe_bench(gpu: Compute, ev: Events, nbytes: int, out_floats: int = 0, laun
     return best
 
 
-PEAK_BF16 = 2.5e15  # MI355X dense bf16 MFMA peak, flop/s
+PEAK_BF16 = 2.5e15  # MI355X dense 16-bit MFMA peak, flop/s
 GEMM_SHAPES = [(Q4_K, 4096, 14336, 128), (Q4_K, 14336, 4096, 128), (Q4_K, 4096, 4096, 128), (Q6_K, 4096, 1024, 128)]
 
 
 def gemm_bench(gpu: Compute, ev: Events, type_: int, cols: int, rows: int, batch: int, launches: int = 20) -> dict:
     """One prompt-batch dequant-GEMM (batch tokens x rows x cols, planar weights) timed with a
     HIP event pair around `launches` back-to-back calls on the library's stream. Algorithmic
-    flops are 2 * batch * rows * cols; the kernel issues three bf16 MFMAs per product (hi/lo
-    operand split), so its MFMA work is three times that."""
+    flops are 2 * batch * rows * cols; the kernel issues two f16 MFMAs per product (hi and lo
+    activations), three for Q6_K (its weights are pairs too), so its MFMA work is that many times more."""
     rng = np.random.default_rng(cols * 5 + rows)
     gen = synth.microbench_q4k if type_ == Q4_K else synth.microbench_q6k
     w = gpu.upload_weights(type_, cols, rows, gen(rng, rows, cols), "gemm w")
@@ -241,8 +241,9 @@ def gemm_bench(gpu: Compute, ev: Events, type_: int, cols: int, rows: int, batch
         gpu.destroy(b)
     t = float(np.mean(times))
     flops = 2.0 * batch * rows * cols
+    m = 3 if type_ == Q6_K else 2
     return {"shape": f"{cols}x{rows}", "type": QUANTS[type_]["name"], "batch": batch, "us": t * 1e6,
-            "tflops": flops / t / 1e12, "mfma_tflops": 3 * flops / t / 1e12, "mfma_frac": 3 * flops / t / PEAK_BF16}
+            "tflops": flops / t / 1e12, "mfma_tflops": m * flops / t / 1e12, "mfma_frac": m * flops / t / PEAK_BF16}
 
 
 def cpu_model() -> str:
@@ -420,7 +421,7 @@ def main() -> None:
         for sh in GEMM_SHAPES:
             g = gemm_bench(gpu, ev, *sh)
             print(f"[bench] gemm {g['type']} {g['shape']} x {g['batch']} tokens: {g['us']:.1f} us, {g['tflops']:.0f} TFLOP/s "
-                  f"({g['mfma_tflops']:.0f} TFLOP/s of bf16 MFMA, {100 * g['mfma_frac']:.1f}% of peak)", file=sys.stderr, flush=True)
+                  f"({g['mfma_tflops']:.0f} TFLOP/s of f16 MFMA, {100 * g['mfma_frac']:.1f}% of peak)", file=sys.stderr, flush=True)
         gpu.dispose()
         return
     wl = WORKLOADS[a.model]
@@ -557,7 +558,7 @@ def main() -> None:
                   f"({100 * m['frac']:.1f}% of 8 TB/s)", file=sys.stderr, flush=True)
         for g in gm:
             print(f"[bench] gemm {g['type']} {g['shape']} x {g['batch']} tokens: {g['us']:.1f} us, {g['tflops']:.0f} TFLOP/s "
-                  f"({100 * g['mfma_frac']:.1f}% of bf16 MFMA peak)", file=sys.stderr, flush=True)
+                  f"({100 * g['mfma_frac']:.1f}% of f16 MFMA peak)", file=sys.stderr, flush=True)
     if not a.no_cpu:
         result["cpu_baseline"] = cpu_baseline(f, wl["title"])
         print(f"[bench] cpu baseline {result['cpu_baseline']['value']:.3f} tok/s", file=sys.stderr, flush=True)

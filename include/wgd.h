@@ -100,7 +100,7 @@ int wgd_done(wgd_context *ctx);
  * for r < rows, b < batch. W holds GGUF blocks of `type` (rows x cols, row-major,
  * quantized along cols). Batch 1 runs the decode matvec (wgd_quantize + wgd_matvec) where
  * the type and layout allow it; batches above 4, and any batch on planar weights, run the
- * dequant-GEMM on bf16 MFMA with a split-precision activation operand; the rest runs a
+ * dequant-GEMM on 16-bit MFMA with a split-precision activation operand; the rest runs a
  * generic f32 kernel. */
 int wgd_matmul(wgd_context *ctx, int32_t type, const wgd_buffer *w, const wgd_buffer *x,
                wgd_buffer *y, uint32_t cols, uint32_t rows, uint32_t stride, uint32_t row_base,

@@ -286,8 +286,8 @@ def test_attention_row_slices(gpu, heads, kvh, hd, start, batch, window, capacit
 
 # Prompt batches (the matrix-core path for head_dim 64/128/256): causal from position 0,
 # a batch deep in the context, a ragged batch with one query head per KV head, a sliding
-# window shorter than the batch's key range, and a wrapped ring. The last two split the
-# keys 7 and 15 ways (the merge's 8- and 16-split forms; the others merge at most 4).
+# window shorter than the batch's key range, and a wrapped ring. The last two split
+# the keys 4 and 8 ways (eight slices of one head per workgroup, a 16-key block each).
 @pytest.mark.parametrize("heads,kvh,hd,start,batch,window,capacity", [
     (32, 8, 128, 0, 128, 4096, 1024), (32, 8, 128, 384, 128, 4096, 1024), (8, 8, 64, 100, 37, 4096, 256),
     (16, 2, 256, 50, 20, 24, 128), (8, 2, 128, 1000, 48, 200, 256), (6, 2, 64, 7, 131, 4096, 512),

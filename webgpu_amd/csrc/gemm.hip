@@ -226,7 +226,7 @@ __global__ __launch_bounds__(256) void k_gemm(GemmArgs a) {
 // ------------------------------------------------------------------ planar quant GEMM
 //
 // The prompt GEMM of the planar layouts (Q4_K, Q5_K, Q6_K, Q8_0, Q4_0; the decode matvec's
-// weights). A workgroup owns QG_M = 128 weight rows x 16 TT tokens and a K span (split-K when
+// weights). A workgroup owns 128 weight rows x 16 TT tokens (256 x 128: TT = 8) and a K span (split-K when
 // the rows alone give too few workgroups; partial sums are added in split order by the
 // finishes, so results do not depend on timing).
 //
@@ -249,9 +249,10 @@ __global__ __launch_bounds__(256) void k_gemm(GemmArgs a) {
 //
 // What it replaces: bf16 pairs of dequantized weights in LDS, always 128 tokens wide, three
 // MFMAs per product and about 210 VALU instructions per 32 weights against about 70. Kernel times
-// of the 8B shape, Q4_K: 16 tokens, gate + up (28672 x 4096) 86 -> 22 us, a prompt of 250
-// tokens in 16s over 4 layers 12.8 -> 6.2 ms; 128 tokens, gate + up 88 -> 83 us, down 47 ->
-// 41, Q/K/V 28.5 -> 27.
+// of the 8B shape, Q4_K: 16 tokens, gate + up (28672 x 4096) 86 -> 20 us (3.3 TB/s of weights), down
+// 47 -> 14, a prompt of 250 tokens in 16s over 4 layers 12.8 -> 5.7 ms; 128 tokens, gate + up 88 ->
+// 78 us (0.77 PFLOP/s of f16 products), down 47 -> 41. At 16 tokens VALU, LDS and MFMA issue add up
+// to about 16 us beside the launch and the first loads; at 128, to the launch: they do not overlap.
 constexpr uint32_t QG_M = 128, QG_K = 64;
 constexpr uint32_t QG_U = SPLIT_K;   // columns of a unit
 
