@@ -284,6 +284,37 @@ def test_attention_row_slices(gpu, heads, kvh, hd, start, batch, window, capacit
         gpu.destroy(b)
 
 
+# A NaN reaches every output that depends on it, however the keys are sliced and split: of the
+# query that holds it, and of every query that sees a key that holds it, also where that key is the only
+# one of its slice. Other outputs are finite.
+@pytest.mark.parametrize("heads,kvh,hd,start,batch", [
+    (4, 1, 128, 0, 20), (2, 2, 64, 0, 33), (8, 1, 64, 0, 17), (32, 8, 128, 240, 10), (2, 2, 128, 1000, 16), (4, 2, 256, 300, 20)])
+def test_prompt_attention_nan(gpu, heads, kvh, hd, start, batch):
+    rng = np.random.default_rng(heads + hd + start)
+    n = start + batch
+    q = rng.standard_normal((batch, heads, hd)).astype(np.float32)
+    k, v = (rng.standard_normal((n, kvh, hd)).astype(np.float32) for _ in range(2))
+    yb = gpu.buffer(q.nbytes, "y")
+    scale = float(1 / np.sqrt(hd))
+    for key in (None, 0, n - 1, start + batch // 2):  # None: a query's NaN
+        qq, kk = q.copy(), k.copy()
+        bad = np.zeros(batch, bool)
+        if key is None:
+            qq[batch // 3] = np.nan
+            bad[batch // 3] = True
+        else:
+            kk[key] = np.nan
+            bad = start + np.arange(batch) >= key
+        bufs = [gpu.upload(a, nm) for a, nm in ((qq, "q"), (kk, "k"), (v, "v"))]
+        gpu.attention(*bufs, yb, heads, kvh, hd, start, scale, 4096, n, n, batch)
+        got = gpu.read_f32(yb, q.size).reshape(q.shape)
+        assert np.isnan(got[bad]).all(), f"NaN of key {key} lost in {int((~np.isnan(got[bad])).sum())} outputs"
+        assert np.isfinite(got[~bad]).all(), f"NaN of key {key} in queries that do not see it"
+        for b in bufs:
+            gpu.destroy(b)
+    gpu.destroy(yb)
+
+
 # Prompt batches (the matrix-core path for head_dim 64/128/256): causal from position 0,
 # a batch deep in the context, a ragged batch with one query head per KV head, a sliding
 # window shorter than the batch's key range, and a wrapped ring. The last two split

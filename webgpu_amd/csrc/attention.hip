@@ -145,8 +145,10 @@ __global__ __launch_bounds__(256) void k_attention(AttnK a) {
   }
 }
 
-// With xs set (hd % 8 == 0, heads * hd % 64 == 0), the output row is also written in the
-// prompt GEMM's split form for the O projection (row = token * heads + head).
+// With xs set (hd % 128 == 0), the output row is also written in the prompt GEMM's split form
+// for the O projection (row = token * heads + head). A split without keys has the sum 0 and is left
+// out; one whose scores are all NaN has the maximum -inf too, but a NaN sum, which has to reach
+// the output.
 __global__ __launch_bounds__(128) void k_attention_combine(const float *part, float *y, uint32_t rows,
                                                            uint32_t hd, uint32_t nsplit, uint8_t *xs, uint32_t heads) {
   __shared__ float out[512];
@@ -157,15 +159,15 @@ __global__ __launch_bounds__(128) void k_attention_combine(const float *part, fl
   float L = 0.f;
   for (uint32_t z = 0; z < nsplit; z++) {
     const float *pp = part + z * stride + row * (hd + 2);
-    if (pp[0] != -INFINITY) L += pp[1] * expf(pp[0] - M);
+    if (pp[1] != 0.f) L += pp[1] * expf(pp[0] - M);
   }
   for (uint32_t d = threadIdx.x; d < hd; d += blockDim.x) {
     float acc = 0.f;
     for (uint32_t z = 0; z < nsplit; z++) {
       const float *pp = part + z * stride + row * (hd + 2);
-      if (pp[0] != -INFINITY) acc += pp[2 + d] * expf(pp[0] - M);
+      if (pp[1] != 0.f) acc += pp[2 + d] * expf(pp[0] - M);
     }
-    const float o = L > 0.f ? acc / L : 0.f;
+    const float o = L == 0.f ? 0.f : acc / L;
     y[row * hd + d] = o;
     out[d] = o;
   }
@@ -202,7 +204,7 @@ __global__ __launch_bounds__(128) void k_attention_combine_s(const float *part, 
   float L = 0.f;
 #pragma unroll
   for (uint32_t z = 0; z < S; z++) {
-    use[z] = z < nsplit && mz[z] != -INFINITY;
+    use[z] = z < nsplit && lz[z] != 0.f;
     wz[z] = use[z] ? expf(mz[z] - M) : 0.f;
     L = use[z] ? L + lz[z] * wz[z] : L;
   }
@@ -214,7 +216,7 @@ __global__ __launch_bounds__(128) void k_attention_combine_s(const float *part, 
     float acc = 0.f;
 #pragma unroll
     for (uint32_t z = 0; z < S; z++) acc = use[z] ? acc + pz[z] * wz[z] : acc;
-    const float o = L > 0.f ? acc / L : 0.f;
+    const float o = L == 0.f ? 0.f : acc / L;
     y[row * hd + d] = o;
     out[d] = o;
   }
@@ -549,7 +551,7 @@ __global__ __launch_bounds__(512) void k_attn_rows(AttnK a, uint32_t hp, uint32_
     for (uint32_t u = 0; u < sl; u++) M = fmaxf(M, lds[(u * hp + hh) * WS + 2 * qi]);
     for (uint32_t u = 0; u < sl; u++) {
       const float *p = lds + (u * hp + hh) * WS;
-      if (p[2 * qi] == -INFINITY) continue;
+      if (p[2 * qi + 1] == 0.f) continue;  // no keys (all NaN: the sum is NaN)
       const float f = expf(p[2 * qi] - M);
       L += p[2 * qi + 1] * f;
       const f32x4 x0 = *(const f32x4 *)(p + 32 + qi * OS + d), x1 = *(const f32x4 *)(p + 32 + qi * OS + d + 4);
@@ -559,7 +561,7 @@ __global__ __launch_bounds__(512) void k_attn_rows(AttnK a, uint32_t hp, uint32_
     const uint32_t head = kv * a.group + h0 + hh;
     const uint64_t row = (uint64_t)tok * a.heads + head;
     if (a.nsplit == 1) {
-      const float inv = L > 0.f ? 1.f / L : 0.f;
+      const float inv = L == 0.f ? 0.f : 1.f / L;
       const float4 ya = make_float4(v[0] * inv, v[1] * inv, v[2] * inv, v[3] * inv);
       const float4 yb = make_float4(v[4] * inv, v[5] * inv, v[6] * inv, v[7] * inv);
       *(float4 *)(a.y + row * HD + d) = ya;
