@@ -257,14 +257,16 @@ def test_attention_long_context_and_ring(gpu, context, start, batch, window, cap
 
 
 # The row-slice kernel (head_dim 64 / 128) at its edges: one query, tiles of
-# 16 ragged and whole, groups that leave wavefronts idle (3) or take two workgroups (12), key
+# 16 ragged and whole, groups that are no power of two, whose workgroups take heads of several query
+# tiles (3, 5, 6, 7, 9, 12) and end with idle wavefronts, key
 # slices that are empty, rings shorter than a block of 16 and rings wrapped inside a block, a window
 # that starts inside a block, 16 key splits, and a ninth query tile of one query. The bound is f32's:
 # sums of up to 3100 keys and 128 products, about 2^-24 * sqrt(keys) of values of order one, with margin.
 @pytest.mark.parametrize("heads,kvh,hd,start,batch,window,capacity", [
     (4, 1, 128, 0, 1, 4096, 64), (3, 1, 64, 5, 2, 4096, 7), (12, 1, 128, 30, 17, 9, 25), (8, 8, 64, 15, 16, 4096, 31),
     (2, 1, 128, 3000, 16, 4096, 3016), (16, 2, 64, 333, 33, 100, 140), (6, 2, 128, 250, 128, 4096, 400),
-    (16, 1, 64, 40, 128, 64, 191), (4, 2, 128, 11, 129, 4096, 256), (32, 8, 128, 240, 10, 4096, 256)])
+    (16, 1, 64, 40, 128, 64, 191), (4, 2, 128, 11, 129, 4096, 256), (32, 8, 128, 240, 10, 4096, 256),
+    (5, 1, 128, 20, 40, 4096, 60), (12, 2, 64, 3, 35, 17, 50), (7, 1, 64, 300, 50, 4096, 350), (9, 1, 128, 10, 33, 4096, 43)])
 @pytest.mark.parametrize("half", [False, True])
 def test_attention_row_slices(gpu, heads, kvh, hd, start, batch, window, capacity, half):
     rng = np.random.default_rng(heads * hd + start + batch)

@@ -433,17 +433,18 @@ __global__ __launch_bounds__(512) void k_attn_rows(AttnK a, uint32_t hp, uint32_
   extern __shared__ float lds[];
   const uint32_t tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c = lane & 15;
   const uint32_t w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const uint32_t kv = blockIdx.x, z = blockIdx.z, hgs = (a.group + hp - 1) / hp;
-  const uint32_t qt = blockIdx.y / hgs, h0 = blockIdx.y % hgs * hp;  // first head of the workgroup in its kv head
+  const uint32_t kv = blockIdx.x, z = blockIdx.z;
+  const uint32_t tiles = (a.batch + 15) / 16 * a.group;  // (query tile, head) pairs of a kv head
+  const uint32_t pair = blockIdx.y * hp + w % hp, qt = pair / a.group;  // this wavefront's
   const uint32_t s0 = a.start_dev ? (uint32_t)*a.start_dev : a.start;
   // the query tile's keys, in blocks of 16, and this wavefront's slice of them
   const uint32_t first_end = s0 + qt * 16 + 1, last_end = s0 + min(a.batch, qt * 16 + 16);
   const uint32_t begin0 = first_end - min(first_end, a.window);
   const uint32_t blocks = (last_end - begin0 + 15) / 16, slices = sl * a.nsplit, per = (blocks + slices - 1) / slices;
   const uint32_t lo = begin0 + 16 * per * (z * sl + w / hp), hi = min(lo + 16 * per, last_end);
-  const uint32_t hw = h0 + w % hp, h = kv * a.group + hw;
+  const uint32_t h = kv * a.group + pair % a.group;
   const uint32_t b = qt * 16 + c;
-  const bool row_ok = hw < a.group && b < a.batch;
+  const bool row_ok = pair < tiles && b < a.batch;
   const uint32_t end_b = s0 + b + 1, begin_b = end_b - min(end_b, a.window);
   const uint32_t cap = a.capacity;
   auto slot = [&](uint32_t base, uint32_t off) {  // (base + off) % cap for base < cap, off < 16
@@ -456,7 +457,7 @@ __global__ __launch_bounds__(512) void k_attn_rows(AttnK a, uint32_t hp, uint32_
 #pragma unroll
     for (uint32_t e = 0; e < 4; e++) o[x][e] = f32x4{0, 0, 0, 0};
   float m = -INFINITY, l = 0.f;
-  if (hw < a.group && lo < hi) {  // wavefront-uniform
+  if (pair < tiles && lo < hi) {  // wavefront-uniform
     f32x4 qr[NT], kr[NT];
 #pragma unroll
     for (uint32_t t = 0; t < NT; t++)
@@ -545,8 +546,9 @@ __global__ __launch_bounds__(512) void k_attn_rows(AttnK a, uint32_t hp, uint32_
   __syncthreads();
   // the slices in order; eight dimensions of a row per thread
   for (uint32_t i = tid; i < hp * 2 * HD; i += blockDim.x) {
-    const uint32_t d = i % (HD / 8) * 8, qi = i / (HD / 8) % 16, hh = i / (2 * HD), tok = qt * 16 + qi;
-    if (tok >= a.batch || h0 + hh >= a.group) continue;
+    const uint32_t d = i % (HD / 8) * 8, qi = i / (HD / 8) % 16, hh = i / (2 * HD);
+    const uint32_t pr = blockIdx.y * hp + hh, tok = pr / a.group * 16 + qi;
+    if (pr >= tiles || tok >= a.batch) continue;
     float M = -INFINITY, L = 0.f, v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     for (uint32_t u = 0; u < sl; u++) M = fmaxf(M, lds[(u * hp + hh) * WS + 2 * qi]);
     for (uint32_t u = 0; u < sl; u++) {
@@ -558,7 +560,7 @@ __global__ __launch_bounds__(512) void k_attn_rows(AttnK a, uint32_t hp, uint32_
 #pragma unroll
       for (int e = 0; e < 4; e++) { v[e] += x0[e] * f; v[4 + e] += x1[e] * f; }
     }
-    const uint32_t head = kv * a.group + h0 + hh;
+    const uint32_t head = kv * a.group + pr % a.group;
     const uint64_t row = (uint64_t)tok * a.heads + head;
     if (a.nsplit == 1) {
       const float inv = L == 0.f ? 0.f : 1.f / L;
@@ -576,14 +578,21 @@ __global__ __launch_bounds__(512) void k_attn_rows(AttnK a, uint32_t hp, uint32_
   }
 }
 
+// (Query tile, head) pairs of one kv head per workgroup: a power of two, so that the eight wavefronts
+// divide into slices for every group, and the group itself where it is one. Pairs are
+// numbered over the query tiles, so a workgroup of a group that is none takes heads of two tiles
+// and no wavefront is idle (workgroups of one tile's heads left 2 to 4 of 8 idle at
+// groups 3, 5 and 12: 16 kv heads, 3000 keys, 72 queries, group 12: 598 us against 334).
+static uint32_t rows_pairs(uint32_t group) { return group >= 5 ? 8 : group >= 3 ? 4 : group; }
+
 template <uint32_t HD, class E>
 static hipError_t launch_attn_rows(hipStream_t s, AttnK a, const AttnArgs &in, uint32_t nsplit) {
-  const uint32_t nqt = (in.batch + 15) / 16, hp = a.group < 8 ? a.group : 8, sl = 8 / hp;
+  const uint32_t nqt = (in.batch + 15) / 16, hp = rows_pairs(a.group), sl = 8 / hp;
   uint8_t *xs = in.xs && in.hd % SPLIT_K == 0 ? in.xs : nullptr;
   a.nsplit = nsplit;
   lds_opt_in((const void *)k_attn_rows<HD, E>);
-  hipLaunchKernelGGL((k_attn_rows<HD, E>), dim3(in.kv_heads, nqt * ((a.group + hp - 1) / hp), nsplit), dim3(64 * hp * sl),
-                     (32 + 16 * (HD + 4)) * sizeof(float) * hp * sl, s, a, hp, sl, xs);
+  hipLaunchKernelGGL((k_attn_rows<HD, E>), dim3(in.kv_heads, (nqt * a.group + hp - 1) / hp, nsplit), dim3(512),
+                     (32 + 16 * (HD + 4)) * sizeof(float) * 8, s, a, hp, sl, xs);
   WGD_HIP(hipGetLastError());
   if (nsplit > 1) launch_attention_combine(s, (const float *)in.partial, in.y, in.batch * in.heads, in.hd, nsplit, xs, in.heads);
   if (in.xs_written) *in.xs_written = xs != nullptr;
@@ -626,7 +635,7 @@ static bool attn_plan(const AttnArgs &in, uint64_t partial_floats, AttnPlan &p) 
     const uint32_t nqt = (in.batch + 15) / 16;
     p.rows = in.hd <= 128;  // at 256, k_attn_rows' operands would not fit its registers
     if (p.rows) {
-      const uint32_t hp = group < 8 ? group : 8, sl = 8 / hp, wgs = in.kv_heads * nqt * ((group + hp - 1) / hp);
+      const uint32_t hp = rows_pairs(group), sl = 8 / hp, wgs = in.kv_heads * ((nqt * group + hp - 1) / hp);
       // a block of 16 keys per wavefront at least (two, in fewer splits: 8B prompt in 16s 6.00
       // -> 6.16 ms), and eight wavefronts per CU (at hd 64, whose wavefronts hold half as much in
       // flight, 16: 128 heads over 6000 keys, 128 queries, 354 -> 328 us), at most the 16 splits that
