@@ -317,6 +317,30 @@ def test_prompt_attention_nan(gpu, heads, kvh, hd, start, batch):
     gpu.destroy(yb)
 
 
+# The choice between the row-slice kernel, its key splits and the kernel that stages keys in LDS, at
+# head_dim 64 / 128: few keys under many heads (staged, one and several tiles), 144 and 136 workgroups on 256
+# CUs (several splits), a batch whose splits the allocation-free entry point bounds, rounds
+# of workgroups, a window, and a wrapped ring. Both entry points give the same bits.
+@pytest.mark.parametrize("heads,kvh,hd,start,batch,window,capacity", [
+    (128, 16, 128, 2, 37, 4096, 64), (64, 8, 64, 1, 128, 4096, 129), (16, 8, 128, 70, 9, 4096, 96),
+    (32, 16, 128, 900, 144, 4096, 1044), (32, 8, 128, 512, 272, 4096, 784), (128, 16, 64, 300, 96, 50, 180),
+    (96, 8, 128, 200, 200, 4096, 400), (64, 8, 128, 14, 16, 20, 41)])
+def test_prompt_attention_choice(gpu, heads, kvh, hd, start, batch, window, capacity):
+    rng = np.random.default_rng(heads + hd + start + batch)
+    q = rng.standard_normal(batch * heads * hd).astype(np.float32)
+    k, v = (rng.standard_normal(capacity * kvh * hd).astype(np.float32) for _ in range(2))
+    bufs = [gpu.upload(a, nm) for a, nm in ((q, "q"), (k, "k"), (v, "v"))] + [gpu.buffer(q.nbytes, "y"), gpu.buffer(q.nbytes, "y2")]
+    scale = float(1 / np.sqrt(hd))
+    gpu.attention(*bufs[:4], heads, kvh, hd, start, scale, window, capacity, capacity, batch)
+    gpu.attention_noalloc(*bufs[:3], bufs[4], heads, kvh, hd, start, scale, window, capacity, capacity, batch)
+    got, same = gpu.read_f32(bufs[3], q.size), gpu.read_f32(bufs[4], q.size)
+    want = orc.attention(q, k.astype(np.float64), v.astype(np.float64), heads, kvh, hd, start, scale, window, capacity, batch)
+    near(got, want, 2e-5, "prompt attention")  # f32 sums, as for the row slices above
+    assert np.array_equal(got.view(np.uint32), same.view(np.uint32))
+    for b in bufs:
+        gpu.destroy(b)
+
+
 # Prompt batches (the matrix-core path for head_dim 64/128/256): causal from position 0,
 # a batch deep in the context, a ragged batch with one query head per KV head, a sliding
 # window shorter than the batch's key range, and a wrapped ring. The last two split

@@ -11,6 +11,9 @@
 // and the key range is split across workgroups (flash-decoding) so decode at long context
 // spreads over the whole chip. Each split keeps an online-softmax state (m, l, O) and a
 // second kernel merges the splits. Tile size T keeps T*hd = 4096 floats per operand.
+#include <algorithm>
+#include <cmath>
+
 #include "internal.h"
 #include "decode.h"
 #include "attention.h"
@@ -243,8 +246,8 @@ static void launch_attention_combine(hipStream_t s, const float *part, float *y,
     hipLaunchKernelGGL(k_attention_combine, dim3(rows), dim3(128), 0, s, part, y, rows, hd, nsplit, xs, heads);
 }
 
-// Prompt batches at head dim 256 on the f32 matrix cores (v_mfma_f32_16x16x4_f32: f32 products,
-// f32 sums, as the f32 shader computes them). A wavefront owns 16 consecutive queries of one head; the
+// Prompt batches on the f32 matrix cores (v_mfma_f32_16x16x4_f32: f32 products, f32 sums, as the
+// f32 shader computes them), at head dim 256 and, where attn_plan picks it over k_attn_rows, 64 and 128. A wavefront owns 16 consecutive queries of one head; the
 // four wavefronts of a workgroup share one kv head and stage 64-key tiles of K (row-major)
 // and V (transposed) in LDS. Scores are formed transposed, S^T = K Q^T, so lane (g, c) holds
 // keys 4g..4g+3 of query row c: a row's running max and sum live in its own lanes (two
@@ -408,17 +411,17 @@ static hipError_t launch_attn_prompt(hipStream_t s, AttnK a, const AttnArgs &in,
 }
 
 // Prompt batches at head dims 64 and 128. k_attn_prompt stages 64-key tiles of K and V through
-// LDS for four (head, query tile) rows, with two barriers and a chain of 256 f32 MFMAs (4096
+// LDS for four (head, query tile) pairs, with two barriers and a chain of 256 f32 MFMAs (4096
 // cycles) per tile and few wavefronts where the batch is small. Here each wavefront owns one
 // head's 16 queries and a slice of the keys, reads K and V straight into the MFMA operands (the
 // heads of a kv head share the lines in their CU's cache) and meets no barrier until the slices of
 // its workgroup merge in LDS; a launch of one key split writes the finished output and its
 // split form. Against k_attn_prompt at these head dims (us, merge included):
 //   32 heads, 16 kv heads, 8191 keys, 16 queries, f32: 99 -> 47 (134 MB of K and V: 2.8 TB/s)
-//   32 / 8 heads, 4000 keys, 32 queries: 65 -> 42; 128 queries, f16: 131 -> 113
-//   16 / 16 heads, 2000 keys, 128 queries: 53 -> 43; 256 queries: 80 -> 70
-//   16 / 8 heads, 64 keys, 64 queries: 15.1 -> 12.4; 2 / 2 heads, 9000 keys, 20 queries: 134 -> 27
-// and no slower at any shape tried (32 / 8 heads, 2000 keys, 512 queries: 232 -> 229). The f32
+//   32 / 8 heads, 4000 keys, 32 queries: 65 -> 42; 128 queries, f16: 133 -> 114
+//   16 / 16 heads, 2000 keys, 128 queries: 53 -> 43; 2 / 2 heads, 9000 keys, 20 queries: 134 -> 27
+// and the other way round where few keys meet many heads (rows_us has both sides): 128 / 16 heads, 39 keys,
+// 37 queries 12.2 against 19.1; 64 / 8 heads, 129 keys, 128 queries, hd 64 18.2 against 25.9. The f32
 // MFMAs bound the long ones: 64 per 16 keys, query tile and head, 2048 cycles.
 // One slice holds whole 16-key blocks:
 //   S^T = K Q^T: lane (g, c) loads 16-byte pieces d = 16 t + 4 g of key c, and holds the
@@ -606,11 +609,56 @@ static uint32_t tile_keys(uint32_t hd) {
   return t;
 }
 
+// Estimated times (us) of the prompt kernels at head dims 64 and 128, by which attn_plan picks one and its key
+// splits n. A CU takes q = ceil(workgroups / CUs) workgroups, as many at once as fit it; a 16-key block of
+// one lasts a latency plus a share for every workgroup at once, and the merge of n > 1 splits a launch
+// and the partials' way through memory. Where the workgroups come in several rounds, the mean over
+// the query tiles counts, else the tile with the most keys. The constants are least-squares fits over 920
+// random shapes (1 to 12000 keys, 1 to 500 queries, 1 to 16 heads per kv head, 1 to 32 kv heads;
+// k_attn_rows with 1 to 16 splits): 13% rms for k_attn_rows, 6% for k_attn_prompt.
+// k_attn_rows reads K and V once per head and query tile and starts and merges eight wavefronts, which
+// few keys under many heads do not pay for (37 queries behind 2 keys, 16 kv heads of 8: 19.1 us against
+// 12.2). Over those shapes it took 0.85 of k_attn_prompt's time on average and up to 1.8 of it alone, in
+// CUs / workgroups splits rounded down (144 queries behind 8000 keys, 16 kv heads of 2, 144 workgroups
+// on 256 CUs: 402 us in one split, 264 in several); the choice takes 0.81, and more than 1.06 at 1% of them.
+static double attn_mb(const AttnArgs &in) { return 4e-6 * in.batch * in.heads * (in.hd + 2); }  // one split's partials
+static double rows_us(const AttnArgs &in, uint32_t keys, uint32_t pairs, uint32_t hp, uint32_t n) {
+  const bool d64 = in.hd == 64;
+  const uint32_t cus = (uint32_t)device_cu_count(), cap = d64 ? 2 : 1, slices = 8 / hp * n;
+  const uint64_t q = ((uint64_t)in.kv_heads * ((pairs + hp - 1) / hp) * n + cus - 1) / cus;
+  auto blocks = [&](uint32_t k) { return (double)(((k + 15) / 16 + slices - 1) / slices); };  // of a wavefront
+  const double last = blocks(keys), per = q > cap && in.batch > 16 ? (last + blocks(keys - in.batch + 16)) / 2 : last;
+  // the share of the eight wavefronts that has keys, in the fullest workgroup
+  const double act = std::min(pairs, hp) * std::min(8.0 / hp, std::ceil((double)((keys + 15) / 16) / per)) / 8;
+  auto block = [&](uint64_t m) { return m ? d64 ? 0.89 + 1.19 * (double)m * act : 0.49 + 2.86 * (double)m * act : 0; };
+  return (d64 ? 4.1 + 0.65 * act : 3.6 + 3.6 * act + 0.25 * attn_mb(in)) +
+         per * ((double)(q / cap) * block(cap) + block(q % cap)) +
+         (n > 1 ? d64 ? 2.5 + 0.6 * n * attn_mb(in) : 1.3 + 0.62 * n * attn_mb(in) : 0);
+}
+static double prompt_us(const AttnArgs &in, uint32_t keys, uint32_t wgs, uint32_t n) {
+  const bool d64 = in.hd == 64;
+  const uint32_t cus = (uint32_t)device_cu_count(), cap = d64 ? 4 : 2;
+  auto tiles = [&](uint32_t k) { return ((k + AP_T - 1) / AP_T + n - 1) / n; };  // of a split
+  auto blocks = [&](uint32_t k) { return std::min(4 * tiles(k), (k + 15) / 16); };
+  const uint64_t q = ((uint64_t)wgs * (((keys + AP_T - 1) / AP_T + tiles(keys) - 1) / tiles(keys)) + cus - 1) / cus;
+  double t = tiles(keys), b = blocks(keys);
+  if (q > cap && in.batch > 16) {
+    t = (t + tiles(keys - in.batch + 16)) / 2;
+    b = (b + blocks(keys - in.batch + 16)) / 2;
+  }
+  auto body = [&](uint64_t m) {
+    return m ? d64 ? 2.5 * t + (0.36 + 0.42 * (double)m) * b : (2.2 + 0.31 * (double)m) * t + 1.21 * (double)m * b : 0;
+  };
+  return (d64 ? 2.4 : 4.2 + 0.42 * attn_mb(in)) + (double)(q / cap) * body(cap) + body(q % cap) +
+         (n > 1 ? (d64 ? 2.3 + 0.95 * n * attn_mb(in) : 2.4 + 0.71 * n * attn_mb(in)) + (n > 16 ? 0.83 * n : 0) : 0) +
+         (n == 1 && in.xs && in.hd % SPLIT_K == 0 ? 2.5 : 0);  // the k_gemm_split launch that k_attn_rows and the merges save
+}
+
 uint64_t attention_scratch_floats(uint32_t heads, uint32_t hd, uint32_t batch, uint32_t max_splits) {
   return (uint64_t)max_splits * batch * heads * (hd + 2);
 }
 
-// How a launch runs: the MFMA kernels (k_attn_rows at hd 64/128, k_attn_prompt at 256, with
+// How a launch runs: the MFMA kernels (k_attn_rows or k_attn_prompt at hd 64/128, k_attn_prompt at 256, with
 // 16-byte aligned operands) or
 // the generic one (query blocks of qb tokens, tiles of T keys), and the number of key
 // chunks: as many as fill the chip, fewer when `partial_floats` holds fewer partials.
@@ -633,21 +681,25 @@ static bool attn_plan(const AttnArgs &in, uint64_t partial_floats, AttnPlan &p) 
   if (aligned && (in.hd == 64 || in.hd == 128 || in.hd == 256)) {
     p.mfma_hd = in.hd;
     const uint32_t nqt = (in.batch + 15) / 16;
-    p.rows = in.hd <= 128;  // at 256, k_attn_rows' operands would not fit its registers
-    if (p.rows) {
-      const uint32_t hp = rows_pairs(group), sl = 8 / hp, wgs = in.kv_heads * ((nqt * group + hp - 1) / hp);
-      // a block of 16 keys per wavefront at least (two, in fewer splits: 8B prompt in 16s 6.00
-      // -> 6.16 ms), and eight wavefronts per CU (at hd 64, whose wavefronts hold half as much in
-      // flight, 16: 128 heads over 6000 keys, 128 queries, 354 -> 328 us), at most the 16 splits that
-      // the merge loads at once. Rounded down, so the partials never outgrow 16 * 8 rows per
-      // workgroup in flight.
-      tiles = ((keys + 15) / 16 + sl - 1) / sl;
-      want = (uint32_t)device_cu_count() * (in.hd == 64 ? 2 : 1) / wgs;
-      if (want > 16) want = 16;
-    } else {
-      const uint32_t wgs = in.kv_heads * ((nqt * group + 3) / 4);
-      tiles = (keys + AP_T - 1) / AP_T;
-      want = ((uint32_t)device_cu_count() * 2 + wgs - 1) / wgs;  // two workgroups per CU: a second wavefront per SIMD
+    // k_attn_prompt: two workgroups per CU, a second wavefront per SIMD
+    const uint32_t wgs = in.kv_heads * ((nqt * group + 3) / 4);
+    tiles = (keys + AP_T - 1) / AP_T;
+    want = ((uint32_t)device_cu_count() * 2 + wgs - 1) / wgs;
+    if (in.hd <= 128) {  // at 256, k_attn_rows' operands would not fit its registers
+      const uint32_t hp = rows_pairs(group), pairs = nqt * group;
+      const uint32_t np = std::max(1u, std::min(tiles, want)), blocks = (keys + 15) / 16;
+      // at most the 16 splits that the merge loads at once, a block per wavefront, and no more partials than
+      // there is room for, in the allocation-free entry point too (the two plan alike)
+      const uint64_t fit = std::min(partial_floats, ATT_NOALLOC_FLOATS) / ((uint64_t)in.batch * in.heads * (in.hd + 2));
+      uint32_t best = 1;
+      double us = rows_us(in, keys, pairs, hp, 1);
+      for (uint32_t n = 2; n <= 16 && 8 / hp * (n - 1) < blocks && n <= fit; n++) {
+        const double t = rows_us(in, keys, pairs, hp, n);
+        if (t < us) { us = t; best = n; }
+      }
+      // (past 128 queries the estimate of k_attn_rows is too short by up to 20% where the keys are few)
+      p.rows = us < (in.batch > 128 ? 0.9 : 1.0) * prompt_us(in, keys, wgs, np) || (np > 1 && np > fit);
+      if (p.rows) tiles = want = best;
     }
   } else {
     p.qb = group >= 16 ? 1 : 16 / group;
@@ -687,6 +739,8 @@ hipError_t attention(hipStream_t s, const AttnArgs &in) {
   a.group = in.heads / in.kv_heads;
   AttnPlan p;
   if (!attn_plan(in, in.partial ? in.partial_floats : 0, p)) return hipErrorInvalidValue;
+  if (!p.rows && p.mfma_hd == 64) return in.kv16 ? launch_attn_prompt<64, _Float16>(s, a, in, p.nsplit) : launch_attn_prompt<64, float>(s, a, in, p.nsplit);
+  if (!p.rows && p.mfma_hd == 128) return in.kv16 ? launch_attn_prompt<128, _Float16>(s, a, in, p.nsplit) : launch_attn_prompt<128, float>(s, a, in, p.nsplit);
   if (p.rows && in.hd == 64) return in.kv16 ? launch_attn_rows<64, _Float16>(s, a, in, p.nsplit) : launch_attn_rows<64, float>(s, a, in, p.nsplit);
   if (p.rows) return in.kv16 ? launch_attn_rows<128, _Float16>(s, a, in, p.nsplit) : launch_attn_rows<128, float>(s, a, in, p.nsplit);
   if (p.mfma_hd == 256) return in.kv16 ? launch_attn_prompt<256, _Float16>(s, a, in, p.nsplit) : launch_attn_prompt<256, float>(s, a, in, p.nsplit);

@@ -201,6 +201,8 @@ struct AttnArgs {
   uint8_t *xs = nullptr; bool *xs_written = nullptr;
   bool kv16 = false;
 };
+// Partial sums that the allocation-free entry point has room for.
+constexpr uint64_t ATT_NOALLOC_FLOATS = 8ull << 20;
 hipError_t attention(hipStream_t s, const AttnArgs &a);
 // Floats of split-K partials attention() writes for these arguments when its scratch does
 // not limit the split count (0: one split, no scratch used).

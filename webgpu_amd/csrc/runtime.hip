@@ -514,7 +514,7 @@ int wgd_probe_read(wgd_context *ctx, const wgd_buffer *src, uint64_t bytes, uint
 // device by wgd_create with that device current, and only that address reaches kernels.
 // Calls on one GPU share its copy (overlapping calls from two streams race); every split
 // writes each of its partial rows before the merge reads them, so nothing needs clearing.
-static constexpr uint64_t NOALLOC_SCRATCH_FLOATS = 8ull << 20;  // 32 MiB
+static constexpr uint64_t NOALLOC_SCRATCH_FLOATS = ATT_NOALLOC_FLOATS;  // 32 MiB
 static __device__ __attribute__((used)) __align__(256) float scratch[NOALLOC_SCRATCH_FLOATS];
 static constexpr int SCRATCH_DEVICES = 64;
 static std::mutex g_scratch_mu;
