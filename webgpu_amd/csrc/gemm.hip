@@ -757,17 +757,24 @@ bool gemm_group_ok(const GemmGroup &g, uint32_t batch) {
 // more take 8: workgroups of 256 rows x 128 tokens, which unpack each weight once (28672 x 4096,
 // 128 tokens: Q4_K 93.7 -> 88.2 us, Q6_K 131.5 -> 111.8). Shorter matrices need the smaller
 // workgroups (4096 x 4096: 18.4 against 22.3), and the 32-column types the registers (Q8_0
-// 100 against 122.5).
+// 100 against 122.5). Q6_K, whose two lo halves cost the most to unpack, takes 8 for shorter matrices
+// too where their columns keep five units or more per workgroup: 100 tokens, 5376 x 21504 117 -> 94,
+// 4096 x 14336 72 -> 62 (with 64 tokens both were slower than the former bf16 kernel's 111 and 70); at 5376 x
+// 5376 (3.4 units) 39.7 against 38.7, at 4096 x 4096 (two) 28.9 against 30.8.
 static uint32_t token_blocks(const GemmGroup &g, uint32_t batch) {
   if (batch <= 16) return 1;
   if (batch <= 64) return batch <= 32 ? 2 : 4;
-  uint32_t tiles = 0;
+  uint32_t tiles = 0, tall = 0;  // of 128 and of 256 rows
+  const Matrix &w = *g.job[0].w;
   for (uint32_t j = 0; j < g.n; j++) {
     const int t = g.job[j].w->type;
-    if (t != g.job[0].w->type || t == Q8_0 || t == Q4_0) return 4;
+    if (t != w.type || t == Q8_0 || t == Q4_0) return 4;
     tiles += (g.job[j].w->rows + QG_M - 1) / QG_M;
+    tall += (g.job[j].w->rows + 2 * QG_M - 1) / (2 * QG_M);
   }
-  return 2 * tiles >= (uint32_t)device_cu_count() ? 8 : 4;
+  const uint32_t cus = (uint32_t)device_cu_count();
+  if (2 * tiles >= cus) return 8;
+  return w.type == Q6_K && (uint64_t)tall * split_kblocks(w.cols) >= 5 * cus ? 8 : 4;
 }
 
 // K span per workgroup: splits until the launch fills its workgroup slots, each at least two units, and
