@@ -181,6 +181,35 @@ def test_prompt_gemm_real_shapes(gpu, type_, rows, cols, batch):
         gpu.destroy(buf)
 
 
+def test_matmul_scratch_grows_once_and_fits_the_budget():
+    """An MLP's projections share one scratch allocation; where the budget does not hold its whole
+    step it is the exact size, and its spare part never keeps another allocation from fitting."""
+    from webgpu_amd.gpu import Compute
+    rng = np.random.default_rng(5)
+    hidden, ffn, batch = 1024, 3072, 32
+    up, down = (GEN[Q6_K](rng, hidden * ffn // 256) for _ in range(2))
+    x = rng.standard_normal((batch, hidden)).astype(np.float32)
+    results = []
+    for budget in (None, 12, 32):
+        gpu = Compute(budget).init()
+        try:
+            wu, wd = gpu.upload_weights(Q6_K, hidden, ffn, up), gpu.upload_weights(Q6_K, ffn, hidden, down)
+            xb, hb, yb = gpu.upload(x, "x"), gpu.buffer(batch * ffn * 4, "h"), gpu.buffer(batch * hidden * 4, "y")
+            gpu.matmul(Q6_K, wu, xb, hb, hidden, ffn, ffn, 0, 0, batch)
+            held = gpu.allocated
+            gpu.matmul(Q6_K, wd, hb, yb, ffn, hidden, hidden, 0, 0, batch)
+            if budget is None:
+                assert gpu.allocated == held
+            if budget == 32:  # 33.5 MB: beside the scratch's 16.8 MB these do not fit
+                gpu.buffer(14 << 20, "other")
+                gpu.matmul(Q6_K, wu, xb, hb, hidden, ffn, ffn, 0, 0, batch)
+                gpu.matmul(Q6_K, wd, hb, yb, ffn, hidden, hidden, 0, 0, batch)
+            results.append(gpu.read_f32(yb, batch * hidden))
+        finally:
+            gpu.dispose()
+    assert np.array_equal(results[0], results[1]) and np.array_equal(results[0], results[2])
+
+
 # every token-block count of the GEMM (16, 32, 64, two of 64) and its edges, widths whose last
 # 128-column unit is half full, and rows that end inside a row tile
 @pytest.mark.parametrize("type_,rows,cols", [(Q4_K, 130, 768), (Q5_K, 17, 256), (Q6_K, 144, 1280), (Q8_0, 129, 320),
