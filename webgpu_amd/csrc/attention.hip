@@ -593,9 +593,10 @@ static hipError_t launch_attn_rows(hipStream_t s, AttnK a, const AttnArgs &in, u
   const uint32_t nqt = (in.batch + 15) / 16, hp = rows_pairs(a.group), sl = 8 / hp;
   uint8_t *xs = in.xs && in.hd % SPLIT_K == 0 ? in.xs : nullptr;
   a.nsplit = nsplit;
-  lds_opt_in((const void *)k_attn_rows<HD, E>);
-  hipLaunchKernelGGL((k_attn_rows<HD, E>), dim3(in.kv_heads, (nqt * a.group + hp - 1) / hp, nsplit), dim3(512),
-                     (32 + 16 * (HD + 4)) * sizeof(float) * 8, s, a, hp, sl, xs);
+  constexpr size_t lds = (32 + 16 * (HD + 4)) * sizeof(float) * 8;
+  if (lds > 65536) lds_opt_in((const void *)k_attn_rows<HD, E>);
+  hipLaunchKernelGGL((k_attn_rows<HD, E>), dim3(in.kv_heads, (nqt * a.group + hp - 1) / hp, nsplit), dim3(512), lds, s, a,
+                     hp, sl, xs);
   WGD_HIP(hipGetLastError());
   if (nsplit > 1) launch_attention_combine(s, (const float *)in.partial, in.y, in.batch * in.heads, in.hd, nsplit, xs, in.heads);
   if (in.xs_written) *in.xs_written = xs != nullptr;

@@ -849,9 +849,10 @@ bool gemm_splits_input(const Matrix &w, const GemmScratch *scratch, uint32_t bat
 
 template <int T0, int T1, uint32_t TT>
 static void launch_qgemm_tt(hipStream_t s, dim3 grid, const QGemm &q) {
-  lds_opt_in((const void *)k_gemm_q<T0, T1, TT>);
   constexpr uint32_t S = qg_stage(T0, TT) > qg_stage(T1, TT) ? qg_stage(T0, TT) : qg_stage(T1, TT);
-  hipLaunchKernelGGL((k_gemm_q<T0, T1, TT>), grid, dim3(qg_threads(TT)), 2 * S * TT * SPLIT_BLOCK, s, q);
+  constexpr uint32_t lds = 2 * S * TT * SPLIT_BLOCK;
+  if (lds > 65536) lds_opt_in((const void *)k_gemm_q<T0, T1, TT>);
+  hipLaunchKernelGGL((k_gemm_q<T0, T1, TT>), grid, dim3(qg_threads(TT)), lds, s, q);
 }
 template <int T0, int T1>
 static void launch_qgemm(hipStream_t s, dim3 grid, uint32_t tb, const QGemm &q) {
