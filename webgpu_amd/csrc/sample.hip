@@ -274,9 +274,9 @@ __device__ __forceinline__ void select(SampleLds &L, const uint64_t *cand, uint3
 }
 
 // The token from the slices' candidates; st (optional) receives it as k_argmax_advance would.
-__global__ __launch_bounds__(SMP_T) void k_sample(const float *logits, const uint64_t *cand, const SliceOut *so,
-                                                  uint32_t nslices, uint32_t slice, const SampleParams *prm,
-                                                  SampleParams value, int32_t index, StepState *st, int32_t *out, int32_t *tokens,
+__global__ __launch_bounds__(SMP_T) void k_sample(const uint64_t *cand, const SliceOut *so, uint32_t nslices,
+                                                  uint32_t slice, const SampleParams *prm, SampleParams value,
+                                                  int32_t index, StepState *st, int32_t *out, int32_t *tokens,
                                                   uint32_t cap, int advance) {
   __shared__ SampleLds L;
   const uint32_t tid = threadIdx.x, lane = tid & 63;
@@ -436,8 +436,8 @@ hipError_t sample(hipStream_t s, const float *logits, uint32_t n, const SamplePa
   SliceOut *so = (SliceOut *)((uint8_t *)scratch + cand_bytes(ns, sl));
   hipLaunchKernelGGL(k_sample_local, dim3(ns), dim3(SL_T), 0, s, logits, n, sl, params, value, cand, so);
   WGD_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_sample, dim3(1), dim3(SMP_T), 0, s, logits, (const uint64_t *)cand, (const SliceOut *)so, ns,
-                     sl, params, value, index, st, out, tokens, cap, advance ? 1 : 0);
+  hipLaunchKernelGGL(k_sample, dim3(1), dim3(SMP_T), 0, s, (const uint64_t *)cand, (const SliceOut *)so, ns, sl, params,
+                     value, index, st, out, tokens, cap, advance ? 1 : 0);
   return hipGetLastError();
 }
 
