@@ -233,6 +233,17 @@ def test_prompt_gemm_batch_edges(gpu, type_, rows, cols):
         assert np.all(np.abs(got - want) <= bound), f"{type_} batch {batch}: {np.max(np.abs(got - want) / np.maximum(bound, 1e-30))}"
         for buf in (xb, yb):
             gpu.destroy(buf)
+    # magnitudes whose sums over 32 columns leave f32's range, though their products with the weights do not
+    x = (rng.uniform(2, 3, (17, cols)) * 1e37).astype(np.float32)
+    want = orc.matmul(type_, w, (x * np.float32(1e-30)).ravel(), cols, rows, rows, 0, 0, 17).reshape(17, rows) * 1e30
+    xb, yb = gpu.upload(x, "x"), gpu.buffer(17 * rows * 4, "y")
+    gpu.matmul(type_, wb, xb, yb, cols, rows, rows, 0, 0, 17)
+    got = gpu.read_f32(yb, 17 * rows).reshape(17, rows)
+    fits = np.abs(want) < 3e38
+    assert fits.mean() > 0.5
+    assert np.all(np.abs(got[fits] - want[fits]) <= 1e-5 * 3e37 * 0.5 * cols), "sums past f32's range"
+    for buf in (xb, yb):
+        gpu.destroy(buf)
     # an infinity stays in its token
     x = rng.standard_normal((20, cols)).astype(np.float32)
     x[7, 3] = np.inf

@@ -237,9 +237,9 @@ __global__ __launch_bounds__(256) void k_gemm(GemmArgs a) {
 // f16 integers: sc * q <= 63 * 31 for Q4_K and Q5_K, q for Q8_0 and Q4_0, and sc * (q - 32)
 // as an exact (hi, lo) pair for Q6_K. The activations are split.h's (hi, lo) pairs: two
 // MFMAs per product (three for Q6_K; its lo * lo part is below 2^-22 of the product). A unit's
-// sums are scaled by the row's d and the token's scale in f32, and the K-quants' min term,
-// -dmin * m times the sums of x, is one f32 MFMA (16x16x4: its four K entries are the unit's
-// four chunks). The worst errors against float64 are those of f32 sums (mlp of Q6_K 4096 x
+// sums are scaled by the row's d in f32, the K-quants' min terms, -dmin * m times the sums of x over
+// the token's scale, come from one f32 MFMA (16x16x4: its four K entries are the unit's four chunks) and are added, and
+// the token's scale comes last. The worst errors against float64 are those of f32 sums (mlp of Q6_K 4096 x
 // 14336, 32 tokens: 2.8e-7 relative; bf16 pairs of both operands gave 6.9e-6).
 //
 // The activations go through two LDS buffers of S units: the next S units are loaded into
@@ -565,15 +565,21 @@ __device__ __forceinline__ void gemm_tile(const QGemm &a, const QJob &jb, uint32
             for (uint32_t r = 0; r < RT; r++) p[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh[j], wl[r][j], p[r], 0, 0, 0);
           }
         }
-        if constexpr (W::MIN) {
-          const float xsum = *(const float *)(xb + SPLIT_SUM + 4 * lane);
+        const float xsum = W::MIN ? *(const float *)(xb + SPLIT_SUM + 4 * lane) : 0.f;
 #pragma unroll
-          for (uint32_t r = 0; r < RT; r++) acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(xsum, mn[r], acc[r][t], 0, 0, 0);
+        for (uint32_t r = 0; r < RT; r++) {
+          if constexpr (W::MIN && TT <= 2) {  // the min terms beside the products: a shorter chain, four registers more
+            const f32x4 m = __builtin_amdgcn_mfma_f32_16x16x4f32(xsum, mn[r], zero, 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 4; i++) p[r][i] = fmaf(p[r][i], dr[r][0], m[i]);
+          } else {
+#pragma unroll
+            for (int i = 0; i < 4; i++) p[r][i] *= dr[r][0];
+            if constexpr (W::MIN) p[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(xsum, mn[r], p[r], 0, 0, 0);
+          }
+#pragma unroll
+          for (int i = 0; i < 4; i++) acc[r][t][i] = fmaf(p[r][i], s[i], acc[r][t][i]);
         }
-#pragma unroll
-        for (uint32_t r = 0; r < RT; r++)
-#pragma unroll
-          for (int i = 0; i < 4; i++) acc[r][t][i] = fmaf(p[r][i] * dr[r][0], s[i], acc[r][t][i]);
       } else {
         f32x4 q[RT];
 #pragma unroll

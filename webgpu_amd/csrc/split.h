@@ -11,7 +11,8 @@
 //     the order 0 2 1 3 4 6 5 7: lane 16 g + c of a v_mfma_f32_16x16x32_f16 takes the 16 bytes
 //     at fragment (hl, j) + 16 * lane. The order inside the eight is the one in which a
 //     dword of packed quants unpacks into f16 pairs (bytes 0 and 2, then 1 and 3);
-//   [g][c] f32: the sum of token c's columns 32 g .. + 32 (the min term of the K-quants);
+//   [g][c] f32: the sum of token c's columns 32 g .. + 32 over s (the min term of the K-quants: over s,
+//     because 32 columns of 2^123 or more would overflow, whose products with the weights need not);
 //   [c] f32: token c's s.
 // Producers that already hold a batch of activations (RMSNorm, the GLU) write this form
 // beside their f32 output so the GEMMs that read it need no split pass of their own.
@@ -67,17 +68,19 @@ __device__ __forceinline__ void split_store8(uint8_t *xs, uint32_t cols, uint32_
   m = max(m, row_other<0x4E>(m));   // quad_perm [2,3,0,1]
   m = max(m, row_other<0x141>(m));  // row_half_mirror
   m = max(m, row_other<0x140>(m));  // row_mirror
-  float sum = ((a.x + a.y) + (a.z + a.w)) + ((b.x + b.y) + (b.z + b.w));
-  sum += __uint_as_float(row_other<0xB1>(__float_as_uint(sum)));
-  sum += __uint_as_float(row_other<0x4E>(__float_as_uint(sum)));
   // s = 2^(E - 127 - 14) for the biased exponent E, bounded so that s and 1 / s are normal
   const uint32_t E = min(max(m >> 23, 16u), 254u);
   const float s = __uint_as_float((E - 14u) << 23), inv = __uint_as_float((254u + 14u - E) << 23);
+  a.x *= inv; a.y *= inv; a.z *= inv; a.w *= inv;
+  b.x *= inv; b.y *= inv; b.z *= inv; b.w *= inv;
+  float sum = ((a.x + a.y) + (a.z + a.w)) + ((b.x + b.y) + (b.z + b.w));
+  sum += __uint_as_float(row_other<0xB1>(__float_as_uint(sum)));
+  sum += __uint_as_float(row_other<0x4E>(__float_as_uint(sum)));
   uint32_t h[4], l[4];
-  split2(a.x * inv, a.z * inv, h[0], l[0]);
-  split2(a.y * inv, a.w * inv, h[1], l[1]);
-  split2(b.x * inv, b.z * inv, h[2], l[2]);
-  split2(b.y * inv, b.w * inv, h[3], l[3]);
+  split2(a.x, a.z, h[0], l[0]);
+  split2(a.y, a.w, h[1], l[1]);
+  split2(b.x, b.z, h[2], l[2]);
+  split2(b.y, b.w, h[3], l[3]);
   const uint32_t c = tok % SPLIT_N, kk = k % SPLIT_K, g = kk / 32, j = (kk % 32) / 8;
   uint8_t *t = xs + split_block_at(tok / SPLIT_N, k / SPLIT_K, split_kblocks(cols));
   uint8_t *f = t + ((j * 4 + g) * 16 + c) * 16;
