@@ -44,6 +44,7 @@ def _cases():
     l = rng.standard_normal(200000).astype(np.float32)
     l[5000:9000] = 8
     yield "ties-fill-slices", l, 1.0, 150, 1.0
+    yield "k-one", rng.standard_normal(262144).astype(np.float32), 1.3, 1, 0.4
     yield "one", np.array([-5.0], np.float32), 0.7, 40, 0.9
     yield "fewer-than-k", np.array([1.0, np.nan, 2.0, 2.0, -1.0, np.inf, 0.5], np.float32), 1.2, 40, 0.9
 

@@ -195,18 +195,22 @@ struct SampleLds {
   uint32_t bin, above, ncand, cutoff;
 };
 
+// What select() starts from: the offsets of the slices' candidate lists in one flat range, and an
+// empty histogram.
+__device__ __forceinline__ void select_begin(SampleLds &L, uint32_t nslices) {
+  if (threadIdx.x == 0) {
+    L.offs[0] = 0;
+    for (uint32_t w = 0; w < nslices; w++) L.offs[w + 1] = L.offs[w] + L.counts[w];
+  }
+  for (uint32_t b = threadIdx.x; b < SMP_BINS; b += SMP_T) L.hist[b] = 0;
+}
+
 // The histogram selection of k_sample: the candidates at or above a bin's start that hold the
 // K largest, through put().
 template <class Put>
 __device__ __forceinline__ void select(SampleLds &L, const uint64_t *cand, uint32_t slice, uint32_t nslices, uint32_t K,
                                        Put put) {
   const uint32_t tid = threadIdx.x;
-  // the offsets of the slices' candidate lists in one flat range [0, C)
-  if (tid == 0) {
-    L.offs[0] = 0;
-    for (uint32_t w = 0; w < nslices; w++) L.offs[w + 1] = L.offs[w] + L.counts[w];
-  }
-  for (uint32_t b = tid; b < SMP_BINS; b += SMP_T) L.hist[b] = 0;
   __syncthreads();
   const uint32_t C = L.offs[nslices];
   auto at = [&](uint32_t i) -> uint64_t {  // flat candidate i: binary search over the offsets
@@ -298,6 +302,7 @@ __global__ __launch_bounds__(SMP_T) void k_sample(const uint64_t *cand, const Sl
   if (lane == 0) { L.wsum[wv] = cnt; L.wmax[wv] = best; }
   if (tid == 0) { L.ncand = 0; L.bound = 0; L.cutoff = 0xFFFFFFFFu; }
   __syncthreads();
+  if (p.top_k > nslices) select_begin(L, nslices);  // beside the sums below
   cnt = 0; best = 0;
   for (uint32_t u = 0; u < SMP_T / 64; u++) {
     cnt += L.wsum[u];
@@ -315,12 +320,12 @@ __global__ __launch_bounds__(SMP_T) void k_sample(const uint64_t *cand, const Sl
     }
   };
   int32_t token = -1;
-  if (cnt > 0 && p.temperature == 0.0) {
-    token = (int32_t)comp_index(best);
+  const uint32_t K = p.top_k < cnt ? p.top_k : cnt;
+  if (cnt > 0 && (p.temperature == 0.0 || K == 1)) {
+    token = (int32_t)comp_index(best);  // one candidate is drawn whatever its probability
   } else if (cnt > 0) {
-    const uint32_t K = p.top_k < cnt ? p.top_k : cnt;
     bool gathered = false;
-    if (K <= nslices) {
+    if (p.top_k <= nslices) {
       // the K-th largest best: the one with K - 1 larger (zeros, slices without a finite
       // logit, are below every composite; with fewer than K bests the bound stays 0)
       if (tid < nslices && mine_so.best) {
@@ -343,7 +348,10 @@ __global__ __launch_bounds__(SMP_T) void k_sample(const uint64_t *cand, const Sl
       __syncthreads();
       gathered = L.ncand <= SMP_CAND;
     }
-    if (!gathered) select(L, cand, slice, nslices, K, put);
+    if (!gathered) {
+      if (p.top_k <= nslices) select_begin(L, nslices);
+      select(L, cand, slice, nslices, K, put);
+    }
     // rank sort, descending: the composites are unique, so each one's place is the count of
     // larger ones
     const uint32_t nc = L.ncand < SMP_CAND ? L.ncand : SMP_CAND;
@@ -360,15 +368,18 @@ __global__ __launch_bounds__(SMP_T) void k_sample(const uint64_t *cand, const Sl
     if (tid < K) L.prob[tid] = exp(((double)comp_value(L.cand[tid]) - (double)comp_value(best)) / p.temperature);
     __syncthreads();
     if (tid == 0) {
-      double sum = 0.0;
-      for (uint32_t j0 = 0; j0 < K; j0 += 8) {  // K <= 200, prob and cum hold 256
-        double q[8];
+      double sum = 0.0, q[8];
 #pragma unroll
-        for (uint32_t e = 0; e < 8; e++) q[e] = L.prob[j0 + e];
+      for (uint32_t e = 0; e < 8; e++) q[e] = L.prob[e];
+      for (uint32_t j0 = 0; j0 < K; j0 += 8) {  // K <= 200, prob and cum hold 256
+        double next[8];  // loaded beside the sums of this chunk
+#pragma unroll
+        for (uint32_t e = 0; e < 8; e++) next[e] = L.prob[j0 + 8 + e];
 #pragma unroll
         for (uint32_t e = 0; e < 8; e++) {
           sum += q[e];
           L.cum[j0 + e] = sum;
+          q[e] = next[e];
         }
       }
     }
