@@ -210,6 +210,14 @@ def test_matmul_scratch_grows_once_and_fits_the_budget():
     assert np.array_equal(results[0], results[1]) and np.array_equal(results[0], results[2])
 
 
+def gemm_bound(x, mags):
+    """Largest error of an output whose products' magnitudes sum to S = |x| |W|^T: the f32 sums' rounding
+    is about sqrt(cols) * 2^-24 of S (times four: the K-quants sum d * sc * q and dmin * m apart, each a few
+    times |w|), and 22-bit activations add 2^-21. The loss of either lo half, of the activations or of
+    Q6_K's weights, is 2^-12 of single products and exceeds it many times."""
+    return (4 * x.shape[1] ** 0.5 * 2.0 ** -24 + 2.0 ** -21) * (np.abs(x.astype(np.float64)) @ mags.T)
+
+
 # every token-block count of the GEMM (16, 32, 64, two of 64) and its edges, widths whose last
 # 128-column unit is half full, and rows that end inside a row tile
 @pytest.mark.parametrize("type_,rows,cols", [(Q4_K, 130, 768), (Q5_K, 17, 256), (Q6_K, 144, 1280), (Q8_0, 129, 320),
@@ -217,6 +225,7 @@ def test_matmul_scratch_grows_once_and_fits_the_budget():
 def test_prompt_gemm_batch_edges(gpu, type_, rows, cols):
     rng = np.random.default_rng(rows + cols)
     w = GEN[type_](rng, rows * cols // QUANTS[type_]["block"])
+    mags = np.abs(orc.dequant(w, type_, rows * cols, f32=False).reshape(rows, cols))
     wb = gpu.upload_weights(type_, cols, rows, w)
     for batch in (2, 15, 16, 17, 32, 33, 64, 65, 128, 129):
         # magnitudes far apart between tokens and between columns: the split is scaled per token and 128 columns
@@ -227,9 +236,7 @@ def test_prompt_gemm_batch_edges(gpu, type_, rows, cols):
         xb, yb = gpu.upload(x, "x"), gpu.buffer(batch * rows * 4, "y")
         gpu.matmul(type_, wb, xb, yb, cols, rows, rows, 0, 0, batch)
         got = gpu.read_f32(yb, batch * rows).reshape(batch, rows)
-        # a sum of cols f32 products in any order: cols * 2^-24 of the sum of magnitudes, which
-        # |w| <= 0.5 of these generators bounds by |x| / 2; 22-bit operands add 2^-21 of it
-        bound = (cols * 2.0 ** -24 + 2.0 ** -21) * 0.5 * np.abs(x.astype(np.float64)).sum(1, keepdims=True)
+        bound = gemm_bound(x, mags)
         assert np.all(np.abs(got - want) <= bound), f"{type_} batch {batch}: {np.max(np.abs(got - want) / np.maximum(bound, 1e-30))}"
         for buf in (xb, yb):
             gpu.destroy(buf)
@@ -253,6 +260,28 @@ def test_prompt_gemm_batch_edges(gpu, type_, rows, cols):
     got = gpu.read_f32(yb, 20 * rows).reshape(20, rows)
     assert not np.any(np.isfinite(got[7]))
     near(np.delete(got, 7, 0), np.delete(want, 7, 0), 1e-4, "tokens beside an infinity")
+    for buf in (wb, xb, yb):
+        gpu.destroy(buf)
+
+
+def test_prompt_gemm_outlier_column(gpu):
+    """A column 10^7 times the others whose weights are zero: the activations' scale is per token and 128
+    columns, so the others keep an absolute precision of 2^-39 of the largest (and 22 bits elsewhere)."""
+    rng = np.random.default_rng(77)
+    rows, cols, batch = 48, 384, 20
+    w = GEN[Q8_0](rng, rows * cols // 32).reshape(rows, cols // 32, 34)
+    w[:, 4, 2 + 5] = 0  # column 133
+    w = w.reshape(-1)
+    x = rng.standard_normal((batch, cols)).astype(np.float32)
+    x[:, 133] = 1e7
+    mags = np.abs(orc.dequant(w, Q8_0, rows * cols, f32=False).reshape(rows, cols))
+    assert not mags[:, 133].any()
+    want = orc.matmul(Q8_0, w, x.ravel(), cols, rows, rows, 0, 0, batch).reshape(batch, rows)
+    wb, xb, yb = gpu.upload_weights(Q8_0, cols, rows, w), gpu.upload(x, "x"), gpu.buffer(batch * rows * 4, "y")
+    gpu.matmul(Q8_0, wb, xb, yb, cols, rows, rows, 0, 0, batch)
+    got = gpu.read_f32(yb, batch * rows).reshape(batch, rows)
+    bound = gemm_bound(x, mags) + 2.0 ** -39 * 2 * 1e7 * mags[:, 128:256].sum(1)
+    assert np.all(np.abs(got - want) <= bound), np.max(np.abs(got - want) / bound)
     for buf in (wb, xb, yb):
         gpu.destroy(buf)
 
@@ -385,12 +414,14 @@ def test_prompt_attention_choice(gpu, heads, kvh, hd, start, batch, window, capa
 
 # Prompt batches (the matrix-core path for head_dim 64/128/256): causal from position 0,
 # a batch deep in the context, a ragged batch with one query head per KV head, a sliding
-# window shorter than the batch's key range, and a wrapped ring. The last two split
-# the keys 4 and 8 ways (eight slices of one head per workgroup, a 16-key block each).
+# window shorter than the batch's key range, and a wrapped ring.
 @pytest.mark.parametrize("heads,kvh,hd,start,batch,window,capacity", [
     (32, 8, 128, 0, 128, 4096, 1024), (32, 8, 128, 384, 128, 4096, 1024), (8, 8, 64, 100, 37, 4096, 256),
     (16, 2, 256, 50, 20, 24, 128), (8, 2, 128, 1000, 48, 200, 256), (6, 2, 64, 7, 131, 4096, 512),
-    (4, 4, 64, 400, 16, 4096, 512), (4, 4, 64, 900, 16, 4096, 1024)])
+    (4, 4, 64, 400, 16, 4096, 512), (4, 4, 64, 900, 16, 4096, 1024),
+    # head dim 256, workgroups of four (query tile, head) pairs: groups of 3 and 1 whose workgroups straddle
+    # query tiles and end ragged, key splits over several tiles, and a wrapped ring
+    (6, 2, 256, 7, 131, 4096, 512), (4, 4, 256, 900, 37, 4096, 1024), (3, 1, 256, 150, 70, 90, 160)])
 def test_prompt_attention_batches(gpu, heads, kvh, hd, start, batch, window, capacity):
     rng = np.random.default_rng(start + batch)
     q = rng.standard_normal(batch * heads * hd).astype(np.float32) * 2

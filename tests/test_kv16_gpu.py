@@ -77,7 +77,7 @@ def test_attention_f16kv_long_context_and_ring(gpu, context, start, batch, windo
 # prompt batches: the matrix-core kernel (head_dim 64/128/256) and the generic one (96)
 @pytest.mark.parametrize("heads,kvh,hd,start,batch,window,capacity", [
     (32, 8, 128, 384, 128, 4096, 1024), (16, 2, 256, 50, 20, 24, 128), (8, 2, 64, 1000, 48, 200, 256),
-    (8, 4, 96, 30, 40, 4096, 128)])
+    (8, 4, 96, 30, 40, 4096, 128), (6, 2, 256, 7, 131, 4096, 512), (4, 4, 256, 900, 37, 4096, 1024)])
 def test_prompt_attention_f16kv_batches(gpu, heads, kvh, hd, start, batch, window, capacity):
     rng = np.random.default_rng(start + batch)
     q = rng.standard_normal(batch * heads * hd).astype(np.float32) * 2

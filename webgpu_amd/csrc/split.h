@@ -4,8 +4,10 @@
 // f16 keeps 11 significant bits, so a value is carried as v = s * (hi + lo) with
 // hi = RN_f16(v / s) and lo = RN_f16(v / s - hi): about 22 bits together. s is a power of two
 // per token and 128 columns that puts their largest magnitude into [2^14, 2^15), so nothing
-// overflows and small values keep their bits (lo is exact down to 2^-24, 38 bits below the
-// largest). The activations [batch][cols] are stored as blocks of 16 tokens x 128 columns,
+// overflows. The pair's last place is 2^-24 s, at most 2^-38 of the largest: a value below 2^-24 of it
+// keeps fewer than the 16 bits that a bf16 pair kept at any magnitude, and below about 2^-39 becomes zero.
+// Beside the largest one's product that is less than f32's rounding; it counts only where that
+// column's weight is zero. The activations [batch][cols] are stored as blocks of 16 tokens x 128 columns,
 // block (token / 16, k / 128) of SPLIT_BLOCK bytes:
 //   [hl][j][g][c][8] f16: token c's columns 32 g + 8 j .. + 8 of the hi (hl = 0) or lo part, in
 //     the order 0 2 1 3 4 6 5 7: lane 16 g + c of a v_mfma_f32_16x16x32_f16 takes the 16 bytes
@@ -58,7 +60,8 @@ __device__ __forceinline__ void split2(float a, float b, uint32_t &hi, uint32_t 
 
 // Columns k..k+7 (k % 8 == 0) of token tok. The 16 lanes of a row together hold 128 columns:
 // lane % 16 == (k / 8) % 16, with the lanes of columns past `cols` (a multiple of 64) off. The
-// largest magnitude goes over those lanes as exponent bits; infinities and NaN stay what they are.
+// largest magnitude goes over those lanes as exponent bits. An infinity's lo part is NaN (inf - inf), so its
+// token's products are NaN; a NaN stays one.
 __device__ __forceinline__ void split_store8(uint8_t *xs, uint32_t cols, uint32_t tok, uint32_t k, float4 a, float4 b) {
   uint32_t m = 0;
   const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
