@@ -244,15 +244,18 @@ __global__ __launch_bounds__(256) void k_gemm(GemmArgs a) {
 //
 // The activations go through two LDS buffers of S units: the next S units are loaded into
 // registers while the current ones are used, one barrier per S units. D units of weights are
-// in flight per row tile. Every load is issued without a branch around it (past the span it
-// reads through an empty resource), so each wait counts exactly the loads behind it.
+// in flight per row tile. No load has a branch around it (past the span it reads through an empty
+// resource), so each wait counts exactly the loads behind it; only the products of a unit past the span are
+// skipped.
 //
 // What it replaces: bf16 pairs of dequantized weights in LDS, always 128 tokens wide, three
 // MFMAs per product and about 210 VALU instructions per 32 weights against about 70. Kernel times
-// of the 8B shape, Q4_K: 16 tokens, gate + up (28672 x 4096) 86 -> 20 us (3.3 TB/s of weights), down
+// of the 8B shape in the model, Q4_K: 16 tokens, gate + up (28672 x 4096) 86 -> 21 us (3.1 TB/s of weights), down
 // 47 -> 14, a prompt of 250 tokens in 16s over 4 layers 12.8 -> 5.7 ms; 128 tokens, gate + up 88 ->
-// 78 us (0.77 PFLOP/s of f16 products), down 47 -> 41. At 16 tokens VALU, LDS and MFMA issue add up
-// to about 16 us beside the launch and the first loads; at 128, to the launch: they do not overlap.
+// 79 us (0.76 PFLOP/s of f16 products), down 47 -> 41. By its counters, gate + up at 16 tokens spends 41% of
+// a wavefront's life on loads, 32% waiting for an issue slot and 27% issuing, with the matrix cores busy for
+// 18% of the launch; at 128 tokens 33%, 40% and 27%, the matrix cores 38%. 128 tokens need 33 us of LDS
+// reads and 20 us of VALU issue beside 30 us of MFMAs; they add up to the launch rather than overlap.
 constexpr uint32_t QG_M = 128, QG_K = 64;
 constexpr uint32_t QG_U = SPLIT_K;   // columns of a unit
 
@@ -468,16 +471,20 @@ template <> struct QUnit<Q4_0> {
 };
 
 // Row tiles per wavefront. Up to 32 tokens the weight stream is the bound, and eight
-// wavefronts of one row tile (128 registers or less, so four per SIMD) hide its latency better
+// wavefronts of one row tile (84 to 119 registers, so four or five per SIMD; 120 to 140 and three with two
+// types at 32 tokens) hide its latency better
 // than four of two (8B prompt in 16s 6.22 against 6.34 ms); for 64 tokens two row tiles halve
 // the LDS reads of the activations per MFMA.
 constexpr uint32_t qg_rt(uint32_t tt) { return tt <= 2 ? 1 : 2; }
 // Rows per workgroup: 128, and 256 (eight wavefronts) where it takes 128 tokens.
 constexpr uint32_t qg_rows(uint32_t tt) { return tt == 8 ? 2 * QG_M : QG_M; }
 constexpr uint32_t qg_threads(uint32_t tt) { return qg_rows(tt) / 16 / qg_rt(tt) * 64; }
-// Units of weights in flight per row tile (registers), and units of activations per LDS buffer (17 to
-// 34 KB). Two units suffice with eight wavefronts or more a CU; four and eight were slower
+// Units of weights in flight per row tile (registers), and units of activations per LDS buffer (17
+// KB at 16 tokens, 34 at 32 and 64, 68 at 128, where the two buffers leave room for one workgroup per CU).
+// Two units suffice with eight wavefronts or more a CU; four and eight were slower
 // (28672 x 4096 Q4_K, 16 tokens: 20.5, 21.5 and 28.8 us), their registers and prologue cost more.
+// Past 32 tokens the registers are full, and some kernels spill outside their inner products: Q4_K or
+// Q5_K with Q6_K (Q, K and V of the usual mixes) 68 bytes a lane, Q5_K and Q6_K at 128 tokens 16.
 constexpr uint32_t qg_depth(int type, uint32_t tt) { return tt == 8 || (tt == 4 && (type == Q8_0 || type == Q4_0)) ? 1 : 2; }
 constexpr uint32_t qg_stage(int type, uint32_t tt) { return tt >= 4 ? 1 : qg_depth(type, tt); }
 
@@ -701,7 +708,9 @@ __device__ __forceinline__ void glu_finish8(const float *part, uint32_t splits, 
 //
 // The GEMM's 128-row tile t ran on XCD t % 8 (its grid's first dimension, the tile count, is
 // a multiple of 8, and workgroups go to the XCDs round-robin), and with R a multiple of 1024
-// the up tile of a column has the gate tile's residue. Then (by_xcd) workgroup w, on XCD
+// the up tile of a column has the gate tile's residue. (Of 256-row workgroups gemm_tile places whole groups
+// of eight per matrix so; the runs of a last group of fewer, 8 of 168 at R = 21504, are read from other
+// XCDs' partials.) Then (by_xcd) workgroup w, on XCD
 // w % 8, takes token w / 8 and the columns of the tiles t = w (mod 8), reading only
 // partials its XCD wrote: each 128-row run of the scratch stays with one XCD, and the next
 // GEMM's writes to it take no coherence probes. Otherwise workgroup w takes 256
@@ -760,8 +769,9 @@ bool gemm_group_ok(const GemmGroup &g, uint32_t batch) {
 
 // 16-token blocks of a workgroup: the smallest of 1, 2, 4 that covers the batch; past 64 tokens
 // workgroups of 64 each. K-quant groups of one type whose 128-row tiles fill half the CUs or
-// more take 8: workgroups of 256 rows x 128 tokens, which unpack each weight once (28672 x 4096,
-// 128 tokens: Q4_K 93.7 -> 88.2 us, Q6_K 131.5 -> 111.8). Shorter matrices need the smaller
+// more take 8: workgroups of 256 rows x 128 tokens, which unpack each weight once (28672 x 4096 as one
+// wgd_matmul over several matrices, 128 tokens: Q4_K 93.7 -> 88.2 us, Q6_K 131.5 -> 111.8; the model's
+// gate + up 79). Shorter matrices need the smaller
 // workgroups (4096 x 4096: 18.4 against 22.3), and the 32-column types the registers (Q8_0
 // 100 against 122.5). Q6_K, whose two lo halves cost the most to unpack, takes 8 for shorter matrices
 // too where their columns keep five units or more per workgroup: 100 tokens, 5376 x 21504 117 -> 94,
