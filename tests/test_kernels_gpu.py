@@ -183,27 +183,32 @@ def test_prompt_gemm_real_shapes(gpu, type_, rows, cols, batch):
 
 def test_matmul_scratch_grows_once_and_fits_the_budget():
     """An MLP's projections share one scratch allocation; where the budget does not hold its whole
-    step it is the exact size, and its spare part never keeps another allocation from fitting."""
+    step it is the exact size, and its spare part never keeps another allocation from fitting.
+    Scratch of at most 2 MiB is of the exact size."""
     from webgpu_amd.gpu import Compute
     rng = np.random.default_rng(5)
-    hidden, ffn, batch = 1024, 3072, 32
+    hidden, ffn, batch = 1024, 8192, 32
     up, down = (GEN[Q6_K](rng, hidden * ffn // 256) for _ in range(2))
     x = rng.standard_normal((batch, hidden)).astype(np.float32)
     results = []
-    for budget in (None, 12, 32):
+    for budget in (None, 24, 36):
         gpu = Compute(budget).init()
         try:
             wu, wd = gpu.upload_weights(Q6_K, hidden, ffn, up), gpu.upload_weights(Q6_K, ffn, hidden, down)
             xb, hb, yb = gpu.upload(x, "x"), gpu.buffer(batch * ffn * 4, "h"), gpu.buffer(batch * hidden * 4, "y")
+            held = gpu.allocated
+            gpu.matmul(Q6_K, wu, xb, hb, hidden, ffn, ffn, 0, 0, 2)
+            assert gpu.allocated - held < 4 << 20
             gpu.matmul(Q6_K, wu, xb, hb, hidden, ffn, ffn, 0, 0, batch)
             held = gpu.allocated
             gpu.matmul(Q6_K, wd, hb, yb, ffn, hidden, hidden, 0, 0, batch)
             if budget is None:
                 assert gpu.allocated == held
-            if budget == 32:  # 33.5 MB: beside the scratch's 16.8 MB these do not fit
+            if budget == 36:  # 37.7 MB: beside the scratch's 16.8 MB these do not fit
                 gpu.buffer(14 << 20, "other")
                 gpu.matmul(Q6_K, wu, xb, hb, hidden, ffn, ffn, 0, 0, batch)
                 gpu.matmul(Q6_K, wd, hb, yb, ffn, hidden, hidden, 0, 0, batch)
+            gpu.matmul(Q6_K, wu, xb, hb, hidden, ffn, ffn, 0, 0, 2)
             results.append(gpu.read_f32(yb, batch * hidden))
         finally:
             gpu.dispose()

@@ -619,9 +619,9 @@ static uint32_t tile_keys(uint32_t hd) {
 // k_attn_rows with 1 to 16 splits): 13% rms for k_attn_rows, 6% for k_attn_prompt.
 // k_attn_rows reads K and V once per head and query tile and starts and merges eight wavefronts, which
 // few keys under many heads do not pay for (37 queries behind 2 keys, 16 kv heads of 8: 19.1 us against
-// 12.2). Over those shapes it took 0.85 of k_attn_prompt's time on average and up to 1.8 of it alone, in
+// 12.2). Over those shapes it took 0.87 of k_attn_prompt's time on average and up to 2.1 of it alone, in
 // CUs / workgroups splits rounded down (144 queries behind 8000 keys, 16 kv heads of 2, 144 workgroups
-// on 256 CUs: 402 us in one split, 264 in several); the choice takes 0.81, and more than 1.06 at 1% of them.
+// on 256 CUs: 402 us in one split, 264 in several); the choice takes 0.81, and more than 1.06 at 2% of them.
 static double attn_mb(const AttnArgs &in) { return 4e-6 * in.batch * in.heads * (in.hd + 2); }  // one split's partials
 static double rows_us(const AttnArgs &in, uint32_t keys, uint32_t pairs, uint32_t hp, uint32_t n) {
   const bool d64 = in.hd == 64;

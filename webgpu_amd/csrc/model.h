@@ -24,7 +24,9 @@ struct wgd_context {
   float *noalloc_scratch = nullptr;  // this device's static scratch (wgd_attention_noalloc)
   void *mv_qx = nullptr;              // quantized activation row of wgd_matmul
   uint64_t mv_qx_bytes = 0;
-  uint8_t *gemm_scratch = nullptr;    // wgd_matmul's prompt GEMM: its input split into f16 (hi, lo), then split-K sums
+  void *gemm_small[2] = {};           // wgd_matmul's prompt GEMM: its input split into f16 (hi, lo); split-K sums
+  uint64_t gemm_small_bytes[2] = {};
+  uint8_t *gemm_scratch = nullptr;    // both, once either is large
   uint64_t gemm_scratch_bytes = 0, gemm_scratch_spare = 0;  // spare: past the need it was allocated for
   int32_t *sample_result = nullptr;            // the token of wgd_sample, in pinned host memory
   void *sample_scratch = nullptr;              // its slices' candidates

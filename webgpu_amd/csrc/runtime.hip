@@ -30,8 +30,8 @@ struct wgd_buffer {
   float qx_eps = 0.f;
 };
 
-static constexpr uint64_t GEMM_SCRATCH_STEP = 16 << 20;
 static thread_local std::string g_error;
+static void gemm_scratch_free(wgd_context *ctx);
 static int scratch_setup(int device, float **out);
 
 int wgd::fail(wgd_context *ctx, int code, const char *fmt, ...) {
@@ -51,10 +51,8 @@ int wgd::hip_fail(wgd_context *ctx, hipError_t e, const char *what) {
 int wgd::ctx_alloc(wgd_context *ctx, uint64_t size, const char *label, void **out) {
   size = size < 4 ? 4 : (size + 3) / 4 * 4;
   // wgd_matmul's scratch holds more than it needs: that never keeps an allocation from fitting
-  if (ctx->allocated + size > ctx->limit && ctx->allocated - ctx->gemm_scratch_spare + size <= ctx->limit) {
-    ctx_free(ctx, ctx->gemm_scratch);
-    ctx->gemm_scratch = nullptr; ctx->gemm_scratch_bytes = ctx->gemm_scratch_spare = 0;
-  }
+  if (ctx->allocated + size > ctx->limit && ctx->allocated - ctx->gemm_scratch_spare + size <= ctx->limit)
+    gemm_scratch_free(ctx);
   if (ctx->allocated + size > ctx->limit)
     return fail(ctx, WGD_E_BUDGET, "GPU budget exceeded allocating %s (%llu bytes). Reduce context length or increase the memory budget.",
                 label, (unsigned long long)size);
@@ -78,6 +76,11 @@ void wgd::ctx_free(wgd_context *ctx, void *p) {
   hipFree(p);
   ctx->allocated -= it->second;
   ctx->sizes.erase(it);
+}
+
+static void gemm_scratch_free(wgd_context *ctx) {
+  ctx_free(ctx, ctx->gemm_scratch);
+  ctx->gemm_scratch = nullptr; ctx->gemm_scratch_bytes = ctx->gemm_scratch_spare = 0;
 }
 
 // Checks for a fault raised by earlier asynchronous work.
@@ -264,6 +267,49 @@ int wgd_done(wgd_context *ctx) {
 
 static bool known_type(int t) { return block_size(t) != 0; }
 
+// Scratch of wgd_matmul's prompt GEMM, grown on demand and kept with the context: xs bytes for the split of
+// the input (re-made on every call) and `sums` bytes for split-K partial sums. hipMalloc takes 1 to 45 us up to
+// 2 MiB and 0.25 to 0.5 ms above where it holds no freed block, so two small buffers are of the exact
+// sizes, and beyond that both share one allocation that grows in whole GEMM_SCRATCH_STEPs where
+// the budget holds them: an MLP's gate, up and down projections allocate once. With two exact buffers of any size
+// a new context's first MLP (Q6_K, 4096 x 14336, 32 tokens) took 0.95 ms, now 0.22; later ones take 0.15.
+static constexpr uint64_t GEMM_SCRATCH_SMALL = 2 << 20, GEMM_SCRATCH_STEP = 16 << 20;
+static int gemm_scratch(wgd_context *ctx, uint64_t xs, uint64_t sums, GemmScratch *gs) {
+  const uint64_t at = (xs + 255) / 256 * 256, need = at + sums;
+  if (need > ctx->gemm_scratch_bytes && xs <= GEMM_SCRATCH_SMALL && sums <= GEMM_SCRATCH_SMALL) {
+    const uint64_t want[2] = {xs, sums};
+    for (int i = 0; i < 2; i++) {
+      if (want[i] <= ctx->gemm_small_bytes[i]) continue;
+      ctx_free(ctx, ctx->gemm_small[i]);
+      ctx->gemm_small[i] = nullptr; ctx->gemm_small_bytes[i] = 0;
+      int rc = ctx_alloc(ctx, want[i], i ? "GEMM split sums" : "GEMM split input", &ctx->gemm_small[i]);
+      if (rc) return rc;
+      ctx->gemm_small_bytes[i] = want[i];
+    }
+    gs->xs = (uint8_t *)ctx->gemm_small[0]; gs->xs_bytes = ctx->gemm_small_bytes[0];
+    gs->p = (float *)ctx->gemm_small[1]; gs->floats = ctx->gemm_small_bytes[1] / 4;
+    return WGD_OK;
+  }
+  if (need > ctx->gemm_scratch_bytes) {
+    for (int i = 0; i < 2; i++) {
+      ctx_free(ctx, ctx->gemm_small[i]);
+      ctx->gemm_small[i] = nullptr; ctx->gemm_small_bytes[i] = 0;
+    }
+    gemm_scratch_free(ctx);
+    uint64_t size = (need + GEMM_SCRATCH_STEP - 1) / GEMM_SCRATCH_STEP * GEMM_SCRATCH_STEP;
+    if (ctx->allocated + size > ctx->limit) size = need;
+    int rc = ctx_alloc(ctx, size, "GEMM split sums and input", (void **)&ctx->gemm_scratch);
+    if (rc) return rc;
+    ctx->gemm_scratch_bytes = size;
+    ctx->gemm_scratch_spare = size - need;
+  }
+  if (!ctx->gemm_scratch) return WGD_OK;
+  ctx->gemm_scratch_spare = std::min(ctx->gemm_scratch_spare, ctx->gemm_scratch_bytes - need);
+  gs->xs = ctx->gemm_scratch; gs->xs_bytes = xs;
+  gs->p = (float *)(ctx->gemm_scratch + at); gs->floats = (ctx->gemm_scratch_bytes - at) / 4;
+  return WGD_OK;
+}
+
 int wgd_matmul(wgd_context *ctx, int32_t type, const wgd_buffer *w, const wgd_buffer *x, wgd_buffer *y,
                uint32_t cols, uint32_t rows, uint32_t stride, uint32_t row_base, uint32_t input_offset,
                uint32_t batch) {
@@ -298,30 +344,9 @@ int wgd_matmul(wgd_context *ctx, int32_t type, const wgd_buffer *w, const wgd_bu
     if (rc) return rc;
     return ctx_check(ctx, mv(ctx->stream, m, nullptr, qx_const(q, cols, false, 0.f), (float *)y->ptr + row_base, MV_STORE), "matmul");
   }
-  // The f16 split of the input, re-made on every call, and the split-K partial sums of the prompt
-  // GEMM: one allocation, grown on demand and kept with the context. It grows in whole GEMM_SCRATCH_STEPs
-  // where the budget holds them, so an MLP's gate, up and down projections allocate once: growing to the
-  // exact sizes, two allocations for gate and two for down, a new context's first MLP (Q6_K, 4096 x 14336,
-  // 32 tokens) took 0.95 ms, now 0.22; later ones take 0.15.
-  const uint64_t gx = m.layout == LAYOUT_PLANAR ? gemm_input_bytes(cols, batch) : 0, at = (gx + 255) / 256 * 256;
-  const uint64_t need = at + gemm_split_floats(m, batch) * 4;
-  if (need > ctx->gemm_scratch_bytes) {
-    ctx_free(ctx, ctx->gemm_scratch);
-    ctx->gemm_scratch = nullptr; ctx->gemm_scratch_bytes = ctx->gemm_scratch_spare = 0;
-    uint64_t size = (need + GEMM_SCRATCH_STEP - 1) / GEMM_SCRATCH_STEP * GEMM_SCRATCH_STEP;
-    if (ctx->allocated + size > ctx->limit) size = need;
-    void *p = nullptr;
-    int rc = ctx_alloc(ctx, size, "GEMM split sums and input", &p);
-    if (rc) return rc;
-    ctx->gemm_scratch = (uint8_t *)p; ctx->gemm_scratch_bytes = size;
-    ctx->gemm_scratch_spare = size - need;
-  }
-  ctx->gemm_scratch_spare = std::min(ctx->gemm_scratch_spare, ctx->gemm_scratch_bytes - need);
   GemmScratch gs;
-  if (ctx->gemm_scratch) {
-    gs.xs = ctx->gemm_scratch; gs.xs_bytes = gx;
-    gs.p = (float *)(ctx->gemm_scratch + at); gs.floats = (ctx->gemm_scratch_bytes - at) / 4;
-  }
+  int rc = gemm_scratch(ctx, m.layout == LAYOUT_PLANAR ? gemm_input_bytes(cols, batch) : 0, gemm_split_floats(m, batch) * 4, &gs);
+  if (rc) return rc;
   return ctx_check(ctx, matmul(ctx->stream, m, (const float *)x->ptr, (float *)y->ptr, stride, row_base, input_offset, batch, &gs), "matmul");
 }
 
