@@ -484,7 +484,9 @@ constexpr uint32_t qg_threads(uint32_t tt) { return qg_rows(tt) / 16 / qg_rt(tt)
 // Two units suffice with eight wavefronts or more a CU; four and eight were slower
 // (28672 x 4096 Q4_K, 16 tokens: 20.5, 21.5 and 28.8 us), their registers and prologue cost more.
 // Past 32 tokens the registers are full, and some kernels spill outside their inner products: Q4_K or
-// Q5_K with Q6_K (Q, K and V of the usual mixes) 68 bytes a lane, Q5_K and Q6_K at 128 tokens 16.
+// Q5_K with Q6_K (Q, K and V of the usual mixes) 68 bytes a lane, Q5_K and Q6_K at 128 tokens 16. One
+// unit of Q6_K in flight at 64 tokens spills nothing (208 registers) and is slower: Q, K and V of the 8B
+// widths, 128 tokens, 29.2 against 27.9 us.
 constexpr uint32_t qg_depth(int type, uint32_t tt) { return tt == 8 || (tt == 4 && (type == Q8_0 || type == Q4_0)) ? 1 : 2; }
 constexpr uint32_t qg_stage(int type, uint32_t tt) { return tt >= 4 ? 1 : qg_depth(type, tt); }
 
